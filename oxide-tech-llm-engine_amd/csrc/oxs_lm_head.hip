@@ -10,18 +10,21 @@
 //   tokens x one 32-wide k block, with the quants in the order the matrix
 //   cores read them (one 16-byte load per lane per block) and the 32 scales
 //   permuted to the rows each lane's accumulators hold;
-// - mmvq_q8_0_kernel: per wavefront 32 tokens x 32 batch columns. Each k block
-//   is one v_mfma_i32_32x32x32_i8, giving the exact integer dot of every
-//   (token, column) pair; the float accumulation then follows the reference
+// - mmvq_q8_0_kernel: per wavefront 32 tokens x 32 or 64 batch columns. Each k
+//   block is one v_mfma_i32_32x32x32_i8 per 32 columns, giving the exact integer
+//   dot of every (token, column) pair; the float accumulation then follows the reference
 //   kernel exactly (four accumulators by b % 4, fmaf(d_w * d_x, dot, acc),
 //   then (A0 + A2) + (A1 + A3)), so y is the reference's to the last bit.
 //
 // Bound: HBM (34 bytes per 32 weights, read once; activations and y are small
 // beside them) and, as the batch grows, the VALU's operations per
 // (token, column, block) that the reference's float order needs (convert the
-// integer dot, scale product, fused multiply-add).
+// integer dot, fused multiply-add; the scale product is a second matrix
+// instruction).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "../../include/oxide_sampler.h"
 
@@ -38,19 +41,6 @@ constexpr int kThreads = 256;
 
 __device__ __forceinline__ float half_to_float(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 
-// (float)half(lo or hi 16 bits of w) * x, rounded once, in one v_fma_mix_f32
-// (S0 read as f16, S1 as f32, S2 = 0): the widening is exact, so this equals
-// the multiply after a conversion, except that a zero product is +0; the
-// accumulators start at +0 and a +0 or -0 product leaves them equal.
-template <int HI>
-__device__ __forceinline__ float half_times(uint32_t w, float x) {
-  float d;
-  if constexpr (HI)
-    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(w), "v"(x));
-  else
-    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(d) : "v"(w), "v"(x));
-  return d;
-}
 __device__ __forceinline__ uint16_t float_to_half(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 
 // Row i of the 32 x 32 MFMA output held in register r of a lane in half g
@@ -113,29 +103,74 @@ __global__ __launch_bounds__(kThreads) void pack_q8_0_kernel(const uint8_t* __re
   }
 }
 
-// mmvq_q8_0_cuda_kernel (quant_gemv_standard.cu:425-513) for 32 columns x
-// 128 tokens per workgroup; each wavefront owns one group of 32 tokens. With
-// a batch above 32 columns, the workgroups of one token range sit 8 apart in
-// launch order: workgroups go round-robin over the 8 XCDs, so they run on
-// the same XCD at about the same time and the second reads the weights from
-// that XCD's L2 instead of HBM.
-// - The activations of a group of four k blocks are staged once per
-//   workgroup in LDS (double-buffered, one barrier per group): quants as
-//   [k block][half g][column][16 bytes], scales converted to float.
-// - Each wavefront loads the next group's weights (one 16-byte load per lane
-//   per block, plus 32 bytes of scales) while it computes the current one.
-// Wavefronts past the last token group skip the arithmetic and stores but
-// keep taking part in the staging and the barriers.
-constexpr int kGroupBlocks = 4;  // k blocks per pipeline step (one per accumulator)
+// mmvq_q8_0_cuda_kernel (quant_gemv_standard.cu:425-513) for 32 * TILES
+// columns x 256 tokens per workgroup; each of its eight wavefronts owns one
+// group of 32 tokens and all of the columns, so the weights are read once per
+// column block. With several column blocks, the workgroups of one token range
+// sit 8 apart in launch order: workgroups go round-robin over the 8 XCDs, so
+// they run on the same XCD at about the same time and the later ones read the
+// weights from that XCD's L2 instead of HBM.
+// - Weights go straight to registers, PF groups of four k blocks ahead: a
+//   block's registers are reloaded as soon as its last matrix instruction has
+//   read them.
+// - The activations of a group are staged once per workgroup in LDS
+//   (double-buffered, one barrier per group): quants as
+//   [k block][half g][column][16 bytes], scales as [column][k block].
+// - The scale products d_w * d_x of a 32 x 32 tile are one more matrix
+//   instruction: an outer product of the two half scales (k = 0 of eight, the
+//   others zero). A product of two halves has at most 22 significant bits, so
+//   its f32 value is exact, as the reference's is. It takes 16 vector
+//   instructions per tile and k block off the VALU, which bound this kernel.
+// Wavefronts past the last token group recompute the last one and store
+// nothing.
+//
+// Bound: HBM up to 32 columns (128256 x 4096: 97.4 us at 5 columns, 5.8 TB/s;
+// 105 at 32), then the issue of converts and FMAs, which two wavefronts per SIMD
+// overlap with the loads (64 columns: 122 us, 4.8 TB/s; 128: 208). The kernel
+// before it (32 columns per wavefront, scale products on the VALU, weights one
+// group ahead) took 119, 125, 215 and 397 us. Measured and left out: four
+// wavefronts per workgroup (181 us at 64 columns), two groups staged per barrier
+// (123).
+constexpr int kGroupBlocks = 4;   // k blocks per group (one per accumulator)
+constexpr int kWaves = 8;         // token groups (wavefronts) per workgroup
+constexpr int kMmThreads = 64 * kWaves;
 
-__global__ __launch_bounds__(kThreads) void mmvq_q8_0_kernel(float* __restrict__ y, const uint8_t* __restrict__ wp,
-                                                             const uint8_t* __restrict__ x, uint32_t m, uint32_t nb,
-                                                             uint32_t batch, uint32_t ncb, uint32_t vec_out) {
-  constexpr int TILES = 1;
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// One half scale as the only nonzero entry of a lane's four (w: the half in
+// the low 16 bits, zero above).
+__device__ __forceinline__ v4h lone_half(uint32_t w) {
+  const uint64_t v = w;
+  return __builtin_bit_cast(v4h, v);
+}
+
+// A 32-bit byte offset whose widening stays next to the load that uses it, so
+// that the load takes a scalar base and this offset.
+__device__ __forceinline__ uint32_t local_offset(uint32_t o) {
+  asm("" : "+v"(o));
+  return o;
+}
+__device__ __forceinline__ uint64_t local_offset(uint64_t o) { return o; }
+
+template <int TILES, int PF>
+__global__ __launch_bounds__(kMmThreads, 2) void mmvq_q8_0_kernel(float* __restrict__ y,
+                                                                  const uint8_t* __restrict__ wp,
+                                                                  const uint8_t* __restrict__ x, uint32_t m,
+                                                                  uint32_t nb, uint32_t batch, uint32_t ncb,
+                                                                  uint32_t vec_out) {
   constexpr int COLS = 32 * TILES;
-  __shared__ __align__(16) uint4 s_xq[2][kGroupBlocks][2][COLS];  // quant halves
-  __shared__ float s_xd[2][kGroupBlocks][COLS];                   // scales as float
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  constexpr int PLANE = COLS + 1;  // 16-byte entries per (block, half) plane; the odd one spreads the banks
+  constexpr int XW = COLS * kGroupBlocks * 9;  // dwords of x per group
+  constexpr int XR = (XW + kMmThreads - 1) / kMmThreads;
+  // per group: quants as [k block][half g][column][16 bytes], then the scales
+  // as [k block][column] pairs {half scale, 0}, as the matrix instruction
+  // takes them; after the two buffers, a third of zeros for lanes 32..63's scales
+  constexpr int XD = kGroupBlocks * 2 * PLANE * 4;
+  constexpr int XG = XD + kGroupBlocks * COLS * 2;
+  __shared__ __align__(16) uint32_t s_x[2 * XG + XG];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   // token block tb and column block cb: in each run of 8 * ncb workgroups,
   // workgroup 8 c + i holds token block i of the run and column block c
   uint32_t tb, cb;
@@ -151,43 +186,53 @@ __global__ __launch_bounds__(kThreads) void mmvq_q8_0_kernel(float* __restrict__
       cb = r - (r / ncb) * ncb;
     }
   }
-  const uint32_t tg = tb * kGroupsPerBlock + wave;
-  const bool live = tg < (m + 31u) / 32u;
+  const uint32_t groups = (m + 31u) / 32u;
+  const uint32_t tg = tb * kWaves + wave;
+  const bool live = tg < groups;
   const uint32_t g = lane >> 5, j = lane & 31u;
   const uint32_t c0 = cb * COLS;
   const uint32_t ngroups = nb / kGroupBlocks;
 
-  // staging: thread t < COLS * 4 copies the q8_1 block (column t / 4, block t % 4) of each group
-  const bool stager = tid < (uint32_t)(COLS * kGroupBlocks);
-  const uint32_t st_col = tid / kGroupBlocks, st_kb = tid % kGroupBlocks;
-  const uint8_t* st_src = x + (size_t)min(c0 + st_col, batch - 1u) * nb * kQ81Bytes + (size_t)st_kb * kQ81Bytes;
-  uint32_t xr[9];
-  auto stage_load = [&](uint32_t grp) {
-    if (stager) {
-      const uint32_t* p = (const uint32_t*)(st_src + (size_t)grp * kGroupBlocks * kQ81Bytes);  // 4-byte aligned
+  // staging: dword i of a group's COLS x 36 dwords, for i = tid, tid + 512, ...:
+  // consecutive lanes read consecutive dwords of a column's 144 bytes
+  // (offsets from the column block; 32 bits for 64 columns, which the host
+  // takes only where they suffice)
+  using XOff = std::conditional_t<TILES == 1, uint64_t, uint32_t>;
+  const uint8_t* xc = x + (size_t)c0 * nb * kQ81Bytes;
+  XOff x_src[XR];
+  uint32_t x_dst[XR], x_and[XR], xr[XR];
 #pragma unroll
-      for (int i = 0; i < 9; ++i) xr[i] = p[i];
-    }
+  for (int i = 0; i < XR; ++i) {
+    const uint32_t w = min(tid + (uint32_t)i * kMmThreads, (uint32_t)XW - 1u);
+    const uint32_t col = w / 36u, d = w - col * 36u, b = d / 9u, e = d - b * 9u;
+    x_src[i] = (XOff)min(col, batch - 1u - c0) * nb * kQ81Bytes + d * 4u;  // + 144 per group
+    x_dst[i] = e == 0u ? XD + (b * COLS + col) * 2u
+                       : ((b * 2u + ((e - 1u) >> 2)) * PLANE + col) * 4u + ((e - 1u) & 3u);
+    x_and[i] = e == 0u ? 0xffffu : 0xffffffffu;  // the scale's word without the sum beside it
+  }
+  auto stage_load = [&](uint32_t grp) {
+    const uint8_t* p = xc + (size_t)min(grp, ngroups - 1u) * (kGroupBlocks * kQ81Bytes);
+#pragma unroll
+    for (int i = 0; i < XR; ++i) xr[i] = *(const uint32_t*)(p + local_offset(x_src[i]));  // 4-byte aligned
   };
-  auto stage_store = [&](int buf) {
-    if (stager) {
-      s_xd[buf][st_kb][st_col] = half_to_float((uint16_t)(xr[0] & 0xffffu));
-      s_xq[buf][st_kb][0][st_col] = make_uint4(xr[1], xr[2], xr[3], xr[4]);
-      s_xq[buf][st_kb][1][st_col] = make_uint4(xr[5], xr[6], xr[7], xr[8]);
-    }
+  auto stage_store = [&](uint32_t buf) {  // (threads past the group's dwords repeat its last one)
+#pragma unroll
+    for (int i = 0; i < XR; ++i) s_x[buf * XG + x_dst[i]] = xr[i] & x_and[i];
   };
 
-  const uint8_t* wg = wp + (size_t)(live ? tg : 0u) * nb * kPackedBlock;
-  v4i wa[kGroupBlocks];
-  uint4 ws0[kGroupBlocks], ws1[kGroupBlocks];
-  auto weight_load = [&](uint32_t grp) {
-#pragma unroll
-    for (int q = 0; q < kGroupBlocks; ++q) {
-      const uint8_t* blk = wg + (size_t)(grp * kGroupBlocks + q) * kPackedBlock;
-      wa[q] = *(const v4i*)(blk + 16 * lane);
-      ws0[q] = *(const uint4*)(blk + 1024 + 32 * g);
-      ws1[q] = *(const uint4*)(blk + 1024 + 32 * g + 16);
-    }
+  // weights: this wavefront's tiles are contiguous; lane l's quants at 16 l,
+  // token j's scale at position 16 ((j / 4) % 2) + 4 (j / 8) + j % 4
+  const uint8_t* wg = wp + (size_t)(live ? tg : groups - 1u) * nb * kPackedBlock;
+  const uint32_t q_off = 16u * lane;
+  const uint32_t s_off = 1024u + 2u * (16u * ((j >> 2) & 1u) + 4u * (j >> 3) + (j & 3u));
+  v4i wa[PF][kGroupBlocks];
+  uint32_t ws[PF][kGroupBlocks];
+  auto group_at = [&](uint32_t grp) {
+    return wg + (size_t)min(grp, ngroups - 1u) * (kGroupBlocks * kPackedBlock);
+  };
+  auto weight_load = [&](int set, int q, const uint8_t* at) {
+    wa[set][q] = *(const v4i*)(at + q * kPackedBlock + local_offset(q_off));
+    ws[set][q] = *(const uint16_t*)(at + q * kPackedBlock + local_offset(s_off));
   };
 
   float acc[TILES][kGroupBlocks][16];
@@ -197,47 +242,76 @@ __global__ __launch_bounds__(kThreads) void mmvq_q8_0_kernel(float* __restrict__
     for (int q = 0; q < kGroupBlocks; ++q)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[t][q][r] = 0.0f;
-  const v16i zero = {};
+  const v16i zi = {};
+  const v16f zf = {};
 
   stage_load(0);
+#pragma unroll
+  for (int s = 0; s < PF; ++s)
+#pragma unroll
+    for (int q = 0; q < kGroupBlocks; ++q) weight_load(s, q, group_at((uint32_t)s));
+  // zeros: the scales' second words, which staging never writes, and lanes 32..63's scales
+  for (uint32_t i = tid; i < 2u * kGroupBlocks * COLS; i += kMmThreads)
+    s_x[(i / (kGroupBlocks * COLS)) * XG + XD + (i % (kGroupBlocks * COLS)) * 2u + 1u] = 0u;
+  for (uint32_t i = tid; i < (uint32_t)XG; i += kMmThreads) s_x[2 * XG + i] = 0u;
   stage_store(0);
-  if (live) weight_load(0);
   __syncthreads();
-  for (uint32_t grp = 0; grp < ngroups; ++grp) {
-    const int buf = grp & 1;
-    v4i ca[kGroupBlocks];
-    uint4 cs0[kGroupBlocks], cs1[kGroupBlocks];
+  uint32_t buf = 0;
+  // one group of four k blocks, from weight set s
+  auto group = [&](auto sc, uint32_t grp) {
+    constexpr int s = decltype(sc)::value;
+    stage_load(grp + 1u);
+    const uint8_t* next = group_at(grp + PF);
+    const uint32_t* xg = s_x + buf * XG;
+    const uint32_t* xq = xg + (g * PLANE + j) * 4u;
+    const uint32_t* xd = (g ? s_x + 2 * XG : xg) + XD + 2u * j;
+    // a tile's columns are read from LDS one tile ahead
+    uint4 bq;
+    uint64_t dx;
+    auto tile_read = [&](int q, int t) {
+      bq = *(const uint4*)(xq + (q * 2 * PLANE + 32 * t) * 4);
+      dx = *(const uint64_t*)(xd + (q * COLS + 32 * t) * 2);
+    };
+    tile_read(0, 0);
 #pragma unroll
     for (int q = 0; q < kGroupBlocks; ++q) {
-      ca[q] = wa[q];
-      cs0[q] = ws0[q];
-      cs1[q] = ws1[q];
-    }
-    const bool more = grp + 1 < ngroups;
-    if (more) {
-      stage_load(grp + 1);
-      if (live) weight_load(grp + 1);
-    }
-    if (live) {
+      // the outer product's k = 0 entries are in lanes 0..31
+      const v4h dw = lone_half(g ? 0u : ws[s][q]);
 #pragma unroll
-      for (int q = 0; q < kGroupBlocks; ++q) {
-        const uint32_t sw[8] = {cs0[q].x, cs0[q].y, cs0[q].z, cs0[q].w, cs1[q].x, cs1[q].y, cs1[q].z, cs1[q].w};
+      for (int t = 0; t < TILES; ++t) {
+        const v4i bv = {(int)bq.x, (int)bq.y, (int)bq.z, (int)bq.w};
+        const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa[s][q], bv, zi, 0, 0, 0);
+        const v16f dd = __builtin_amdgcn_mfma_f32_32x32x8f16(dw, __builtin_bit_cast(v4h, dx), zf, 0, 0, 0);
+        if (t + 1 < TILES) tile_read(q, t + 1);
+        else if (q + 1 < kGroupBlocks) tile_read(q + 1, 0);
+        if (t + 1 == TILES) weight_load(s, q, next);  // this block's registers, PF groups ahead
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-          const uint4 bq = s_xq[buf][q][g][32 * t + j];
-          const float dx = s_xd[buf][q][32 * t + j];
-          const v4i bv = {(int)bq.x, (int)bq.y, (int)bq.z, (int)bq.w};
-          const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(ca[q], bv, zero, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float dd = (r % 2) ? half_times<1>(sw[r / 2], dx) : half_times<0>(sw[r / 2], dx);
-            acc[t][q][r] = __builtin_fmaf(dd, (float)d[r], acc[t][q][r]);
-          }
+        for (int r = 0; r < 16; ++r) {
+          acc[t][q][r] = __builtin_fmaf(dd[r], (float)d[r], acc[t][q][r]);
+          asm("" : "+v"(acc[t][q][r]));  // computed here: not put off to the end of the group
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (more) stage_store(buf ^ 1);
+    buf ^= 1u;
+    stage_store(buf);
     __syncthreads();
+  };
+  // (No branch leaves the unrolled groups: with one, the wait before a
+  // register's use would count the loads of the shortest path through the
+  // loop, and the weights would be waited for almost as soon as issued.)
+  uint32_t g0 = 0;
+  for (; g0 + PF <= ngroups; g0 += PF) {
+    group(std::integral_constant<int, 0>{}, g0);
+    if constexpr (PF > 1) group(std::integral_constant<int, 1>{}, g0 + 1u);
+    if constexpr (PF > 2) group(std::integral_constant<int, 2>{}, g0 + 2u);
+    if constexpr (PF > 3) group(std::integral_constant<int, 3>{}, g0 + 3u);
+  }
+  if (g0 < ngroups) group(std::integral_constant<int, 0>{}, g0);
+  if constexpr (PF > 2) {
+    if (g0 + 1u < ngroups) group(std::integral_constant<int, 1>{}, g0 + 1u);
+    if (g0 + 2u < ngroups) group(std::integral_constant<int, 2>{}, g0 + 2u);
   }
   if (!live) return;
 
@@ -268,9 +342,9 @@ __global__ __launch_bounds__(kThreads) void mmvq_q8_0_kernel(float* __restrict__
   }
 }
 
-// The same product for batches of at most four columns, where a 32-column
-// MFMA tile would be mostly idle (eight columns was measured slower than the
-// MFMA kernel). Each workgroup first stages the whole of x
+// The same product for batches of one or two columns, where a 32-column MFMA
+// tile would be almost idle (128256 x 4096: 96.0 and 93.7 us against 97.4 for
+// the MFMA kernel; at four columns it took 103.9). Each workgroup first stages the whole of x
 // (NC columns x every k block) in LDS, then each wavefront walks its 32
 // tokens with no further barrier: lane (j, g) takes 16 quant bytes of token j
 // per block (the packed layout's MFMA order), four dot4 products per column,
@@ -377,28 +451,31 @@ extern "C" int oxs_mmvq_q8_0(float* y, const void* w_packed, const void* x_q8_1,
   const uint32_t vec_out = (m % 4u == 0u && ((uintptr_t)y & 15u) == 0u) ? 1u : 0u;
   const uint32_t groups = (m + 31u) / 32u;
   const uint32_t gx = (groups + oxs_lm::kGroupsPerBlock - 1) / oxs_lm::kGroupsPerBlock;
-  const uint32_t nc_small = batch <= 1u ? 1u : batch <= 2u ? 2u : 4u;  // columns the small kernel stages
-  if (batch <= 4u && (size_t)nc_small * (k / 32u) * 36u <= 65536u) {    // the whole of x fits in LDS
+  if (batch <= 2u && (size_t)batch * (k / 32u) * 36u <= 65536u) {  // the whole of x fits in LDS
     const uint32_t nb = k / 32u;
-    const size_t lds = (size_t)nc_small * nb * 36u;
+    const size_t lds = (size_t)batch * nb * 36u;
     const dim3 g1(gx);
-    switch (batch) {
-      case 1: hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_small_kernel<1>, g1, dim3(oxs_lm::kThreads), lds,
-                                 (hipStream_t)stream, y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb,
-                                 batch); break;
-      case 2: hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_small_kernel<2>, g1, dim3(oxs_lm::kThreads), lds,
-                                 (hipStream_t)stream, y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb,
-                                 batch); break;
-      default: hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_small_kernel<4>, g1, dim3(oxs_lm::kThreads), lds,
-                                  (hipStream_t)stream, y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb,
-                                  batch); break;
-    }
+    if (batch == 1u)
+      hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_small_kernel<1>, g1, dim3(oxs_lm::kThreads), lds, (hipStream_t)stream, y,
+                         (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb, batch);
+    else
+      hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_small_kernel<2>, g1, dim3(oxs_lm::kThreads), lds, (hipStream_t)stream, y,
+                         (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb, batch);
     return launch_status();
   }
-  const uint32_t ncb = (batch + 31u) / 32u;  // 32-column blocks
-  const uint64_t grid = (uint64_t)gx * ncb;
+  // columns per workgroup: 64 halves the weight reads of a larger batch, but
+  // needs offsets into 64 columns of x in 32 bits
+  const uint32_t cols = batch <= 32u || (uint64_t)64u * (k / 32u) * oxs_lm::kQ81Bytes > 0xffffffffull ? 32u : 64u;
+  const uint32_t ncb = (batch + cols - 1u) / cols;
+  const uint64_t grid = (uint64_t)((groups + oxs_lm::kWaves - 1) / oxs_lm::kWaves) * ncb;
   if (grid > 0x7fffffffull) return OXS_ERR_INVALID_ARGUMENT;
-  hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_kernel, dim3((uint32_t)grid), dim3(oxs_lm::kThreads), 0, (hipStream_t)stream,
-                     y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, k / 32u, batch, ncb, vec_out);
+  if (cols == 32u)
+    hipLaunchKernelGGL((oxs_lm::mmvq_q8_0_kernel<1, 4>), dim3((uint32_t)grid), dim3(oxs_lm::kMmThreads), 0,
+                       (hipStream_t)stream, y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, k / 32u, batch,
+                       ncb, vec_out);
+  else
+    hipLaunchKernelGGL((oxs_lm::mmvq_q8_0_kernel<2, 2>), dim3((uint32_t)grid), dim3(oxs_lm::kMmThreads), 0,
+                       (hipStream_t)stream, y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, k / 32u, batch,
+                       ncb, vec_out);
   return launch_status();
 }

@@ -215,8 +215,8 @@ def test_gpu_quantize_matches_oracle(torch_gpu, batch, k):
                                        (129, 4096, 4), (70, 16384, 4), (64, 16384, 5), (257, 4096, 6), (96, 4096, 8),
                                        (40, 8192, 8), (33, 128, 9)])
 def test_gpu_mmvq_matches_oracle(torch_gpu, m, k, batch):
-    # batch <= 4 with x (staged for 1, 2 or 4 columns) within 64 KB of LDS takes the
-    # small-batch kernel; (70, 16384, 4) and batch > 4 take the MFMA kernel
+    # batch <= 2 with x within 64 KB of LDS takes the
+    # small-batch kernel; larger batches take the MFMA kernel
     from oxide_sampler import LmHeadQ8_0, quantize_q8_1
     rng = np.random.default_rng(m + 3 * k + 7 * batch)
     w, x = random_case(rng, m, k, batch)
@@ -226,6 +226,40 @@ def test_gpu_mmvq_matches_oracle(torch_gpu, m, k, batch):
     got = head.project(xq.view(batch, -1)).cpu().numpy()
     want = oracle.mmvq_q8_0_host(w, oracle.quantize_q8_1_host(x), m, k, batch)
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,batch", [
+    (1, 128, 3), (255, 128, 32), (256, 128, 33), (257, 256, 64), (513, 384, 34), (31, 512, 64),
+    (300, 640, 5), (290, 768, 95), (64, 896, 128), (2049, 1024, 129)])
+def test_gpu_mmvq_tiles_and_group_remainders(torch_gpu, m, k, batch):
+    # the edges of the matrix kernel: 32 and 64 columns per workgroup and their remainders, 256
+    # tokens per workgroup, 1 to 8 groups of four k blocks (the prefetch is 4 and 2 groups deep);
+    # scales that are subnormal halves, zero, infinite or NaN, on both sides
+    from oxide_sampler import LmHeadQ8_0
+    rng = np.random.default_rng(m + 5 * k + 11 * batch)
+    w, x = random_case(rng, m, k, batch)
+    nb = k // 32
+    w = w.copy().reshape(m, nb, 34)
+    xq = oracle.quantize_q8_1_host(x).copy().reshape(batch, nb, 36)
+    odd = np.array([0x0001, 0x8001, 0x03FF, 0x83FF, 0x0000, 0x8000, 0x7BFF, 0xFBFF], np.uint16)
+    for blocks, count in ((w, m), (xq, batch)):
+        rows, cols = rng.integers(0, count, 40), rng.integers(0, nb, 40)
+        blocks[rows, cols, :2] = rng.choice(odd, 40).view(np.uint8).reshape(40, 2)
+    xq[:, :, 2:4] = rng.choice(np.array([0x7C00, 0xFC00, 0x7E00, 0x0001], np.uint16),
+                               (batch, nb)).view(np.uint8).reshape(batch, nb, 2)  # the sums are never read
+    w[m - 1, nb - 1, :2] = np.array([0x7C00], np.uint16).view(np.uint8)  # an infinite weight scale
+    if batch > 1:
+        xq[batch - 1, 0, :2] = np.array([0xFC00], np.uint16).view(np.uint8)  # an infinite activation scale
+        xq[0, nb - 1, :2] = np.array([0x7E00], np.uint16).view(np.uint8)  # NaN
+    print(f"\n[case] mmvq_q8_0 edges m={m} k={k} batch={batch}", flush=True)
+    head = LmHeadQ8_0(w.reshape(-1), m, k)
+    got = head.project(_to_dev(torch_gpu, xq.reshape(batch, -1))).cpu().numpy()
+    want = oracle.mmvq_q8_0_host(w.reshape(-1), xq.reshape(-1), m, k, batch)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    np.testing.assert_array_equal(got.view(np.uint32)[ok], want.view(np.uint32)[ok])
+    assert np.isinf(want).any() or batch == 1
 
 
 @pytest.mark.gpu
