@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void pack_q8_0_kernel(const uint8_t* __re
 }
 
 // mmvq_q8_0_cuda_kernel (quant_gemv_standard.cu:425-513) for 32 * TILES
-// columns x 256 tokens per workgroup; each of its eight wavefronts owns one
+// columns x 32 * WAVES tokens per workgroup; each of its wavefronts owns one
 // group of 32 tokens and all of the columns, so the weights are read once per
 // column block. With several column blocks, the workgroups of one token range
 // sit 8 apart in launch order: workgroups go round-robin over the 8 XCDs, so
@@ -128,12 +128,10 @@ __global__ __launch_bounds__(kThreads) void pack_q8_0_kernel(const uint8_t* __re
 // 105 at 32), then the issue of converts and FMAs, which two wavefronts per SIMD
 // overlap with the loads (64 columns: 122 us, 4.8 TB/s; 128: 208). The kernel
 // before it (32 columns per wavefront, scale products on the VALU, weights one
-// group ahead) took 119, 125, 215 and 397 us. Measured and left out: four
-// wavefronts per workgroup (181 us at 64 columns), two groups staged per barrier
-// (123).
+// group ahead) took 119, 125, 215 and 397 us. Measured and left out: 64 columns
+// with four wavefronts per workgroup (they spill; 181 us), two groups staged per
+// barrier (123).
 constexpr int kGroupBlocks = 4;   // k blocks per group (one per accumulator)
-constexpr int kWaves = 8;         // token groups (wavefronts) per workgroup
-constexpr int kMmThreads = 64 * kWaves;
 
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -153,12 +151,14 @@ __device__ __forceinline__ uint32_t local_offset(uint32_t o) {
 }
 __device__ __forceinline__ uint64_t local_offset(uint64_t o) { return o; }
 
-template <int TILES, int PF>
-__global__ __launch_bounds__(kMmThreads, 2) void mmvq_q8_0_kernel(float* __restrict__ y,
+// WAVES: token groups (wavefronts) per workgroup
+template <int TILES, int PF, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void mmvq_q8_0_kernel(float* __restrict__ y,
                                                                   const uint8_t* __restrict__ wp,
                                                                   const uint8_t* __restrict__ x, uint32_t m,
                                                                   uint32_t nb, uint32_t batch, uint32_t ncb,
                                                                   uint32_t vec_out) {
+  constexpr int kMmThreads = 64 * WAVES;
   constexpr int COLS = 32 * TILES;
   constexpr int PLANE = COLS + 1;  // 16-byte entries per (block, half) plane; the odd one spreads the banks
   constexpr int XW = COLS * kGroupBlocks * 9;  // dwords of x per group
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kMmThreads, 2) void mmvq_q8_0_kernel(float* __restr
     }
   }
   const uint32_t groups = (m + 31u) / 32u;
-  const uint32_t tg = tb * kWaves + wave;
+  const uint32_t tg = tb * WAVES + wave;
   const bool live = tg < groups;
   const uint32_t g = lane >> 5, j = lane & 31u;
   const uint32_t c0 = cb * COLS;
@@ -463,19 +463,30 @@ extern "C" int oxs_mmvq_q8_0(float* y, const void* w_packed, const void* x_q8_1,
                          (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb, batch);
     return launch_status();
   }
-  // columns per workgroup: 64 halves the weight reads of a larger batch, but
-  // needs offsets into 64 columns of x in 32 bits
-  const uint32_t cols = batch <= 32u || (uint64_t)64u * (k / 32u) * oxs_lm::kQ81Bytes > 0xffffffffull ? 32u : 64u;
-  const uint32_t ncb = (batch + cols - 1u) / cols;
-  const uint64_t grid = (uint64_t)((groups + oxs_lm::kWaves - 1) / oxs_lm::kWaves) * ncb;
+  // Columns and tokens per workgroup. 64 columns read the weights half as often
+  // as 32 and 256 tokens stage x half as often as 128, but each needs enough
+  // workgroups to occupy the 256 CUs, one per CU; the line lies between 125 and
+  // 197 of them. Measured, us: 64 columns / 32 columns for a batch of 64 at
+  // k = 4096, 125 workgroups (m = 32000) 45.0 / 39.5, 197 (m = 50257) 61.7 / 69.4;
+  // 256 / 128 tokens at a batch of 5, 125 workgroups 30.3 / 25.6, 197 42.2 / 45.6.
+  // (64 columns also need their offsets into x within 32 bits.)
+  constexpr uint64_t kEnough = 160;
+  const uint32_t nb = k / 32u;
+  const auto blocks = [&](uint32_t cols, uint32_t waves) {
+    return (uint64_t)((groups + waves - 1u) / waves) * ((batch + cols - 1u) / cols);
+  };
+  const bool wide = batch > 32u && blocks(64u, 8u) >= kEnough && (uint64_t)64u * nb * oxs_lm::kQ81Bytes <= 0xffffffffull;
+  const uint32_t cols = wide ? 64u : 32u;
+  const uint32_t waves = wide || blocks(32u, 8u) >= kEnough ? 8u : 4u;
+  const uint64_t grid = blocks(cols, waves);
   if (grid > 0x7fffffffull) return OXS_ERR_INVALID_ARGUMENT;
-  if (cols == 32u)
-    hipLaunchKernelGGL((oxs_lm::mmvq_q8_0_kernel<1, 4>), dim3((uint32_t)grid), dim3(oxs_lm::kMmThreads), 0,
-                       (hipStream_t)stream, y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, k / 32u, batch,
-                       ncb, vec_out);
-  else
-    hipLaunchKernelGGL((oxs_lm::mmvq_q8_0_kernel<2, 2>), dim3((uint32_t)grid), dim3(oxs_lm::kMmThreads), 0,
-                       (hipStream_t)stream, y, (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, k / 32u, batch,
-                       ncb, vec_out);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(64u * waves), 0, (hipStream_t)stream, y,
+                       (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb, batch, (batch + cols - 1u) / cols,
+                       vec_out);
+  };
+  if (wide) go(oxs_lm::mmvq_q8_0_kernel<2, 2, 8>);
+  else if (waves == 8u) go(oxs_lm::mmvq_q8_0_kernel<1, 4, 8>);
+  else go(oxs_lm::mmvq_q8_0_kernel<1, 4, 4>);
   return launch_status();
 }

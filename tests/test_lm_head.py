@@ -231,10 +231,11 @@ def test_gpu_mmvq_matches_oracle(torch_gpu, m, k, batch):
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,k,batch", [
     (1, 128, 3), (255, 128, 32), (256, 128, 33), (257, 256, 64), (513, 384, 34), (31, 512, 64),
-    (300, 640, 5), (290, 768, 95), (64, 896, 128), (2049, 1024, 129)])
+    (300, 640, 5), (290, 768, 95), (64, 896, 128), (2049, 1024, 129),
+    (40961, 128, 3), (41217, 256, 33), (20481, 384, 65)])
 def test_gpu_mmvq_tiles_and_group_remainders(torch_gpu, m, k, batch):
-    # the edges of the matrix kernel: 32 and 64 columns per workgroup and their remainders, 256
-    # tokens per workgroup, 1 to 8 groups of four k blocks (the prefetch is 4 and 2 groups deep);
+    # the edges of the matrix kernel's three forms (32 columns x 128 tokens per workgroup; from 160
+    # workgroups 32 x 256, and 64 x 256 for batches above 32) and their remainders, 1 to 8 groups of four k blocks (the prefetch is 4 and 2 groups deep);
     # scales that are subnormal halves, zero, infinite or NaN, on both sides
     from oxide_sampler import LmHeadQ8_0
     rng = np.random.default_rng(m + 5 * k + 11 * batch)
