@@ -5,13 +5,14 @@
 // crates/oxide-server/src/grammar_engine.rs:42-65) and writes the packed
 // allowed-token bitmask that oxs_sample_batch reads (oxs_batch.allowed_mask).
 //
-// One thread per token: its bytes are read kMaxBytes at a time into registers,
-// once, and each piece is walked from every row of the block's row group, whose
-// states stay in registers, four rows interleaved so that four independent
-// table reads are in flight per step. The table sits in LDS when it fits. A walk is a chain of dependent table reads, so the table
-// lookups bound this kernel, not HBM (the token bytes and offsets are read once
-// per row group). A wavefront's 64 consecutive tokens give two mask words per
-// row from one ballot.
+// One thread per token. Its bytes come in 16-byte pieces, and each piece is
+// walked from up to 64 start states (every state of a small table, or the
+// states of 64 rows): a table of the start states that accept each first byte
+// leaves few walks, and tables of up to 8 states compose whole transition
+// functions with byte permutes. The tokens' results are turned into one mask
+// word per start state and 32 tokens, which the rows then copy. Bound: latency
+// (the token bytes and offsets are read once per row group; the masks are
+// written once).
 //
 // A walk depends only on the state it starts from, so a decode loop computes
 // the masks of every state once per grammar and vocabulary (this kernel over
@@ -25,13 +26,13 @@
 namespace oxs_grammar {
 
 constexpr int kThreads = 256;
-constexpr int kTokPerThread = 4;      // tokens per thread (amortises the table's load into LDS)
-constexpr int kRowsPerBlock = 16;     // rows walked per block
-constexpr int kRowIlp = 4;            // rows walked together
-constexpr int kMaxBytes = 16;         // token bytes read and walked per piece
-constexpr uint32_t kLdsStates = 48;   // tables of up to 48 states (48 KB) are copied into LDS
+constexpr int kTok = 2;               // tokens per thread
+constexpr int kWords = kTok * kThreads / 32;  // mask words per row and block
+constexpr int kRows = 128;            // rows per block with a walk from every state
+constexpr uint32_t kList = 64;        // start states walked together
+constexpr uint32_t kPermStates = 8;   // tables whose transition functions fit a byte permute
+constexpr uint32_t kLdsStates = 128;  // tables of up to 128 states are kept in LDS, a byte per entry
 constexpr uint32_t kErr = OXS_DFA_ERROR_STATE;
-static_assert(kRowsPerBlock % kRowIlp == 0, "rows are walked kRowIlp at a time");
 
 struct Params {
   const uint32_t* trans;
@@ -46,193 +47,215 @@ struct Params {
   int64_t mask_ld;
 };
 
-// One transition (DfaSchemaGrammar::transition, dfa.rs:110-126): a current
-// state outside the table or an error entry ends the walk as invalid.
-__device__ __forceinline__ void step(const uint32_t* T, uint32_t ns, uint32_t byte, uint32_t& s, bool& ok) {
-  if (!ok) return;
-  if (s >= ns) {
-    ok = false;
-    return;
-  }
-  s = T[s * 256u + byte];
-  ok = s != kErr;
+// Next states as bytes. With kPermStates states a byte is also a v_perm_b32
+// selector: 0-7 pick a byte of the function, anything from 0x0d up gives 0xff.
+// So a walk that left the table (kOut: allowed if its token ends there) or
+// failed (kDead) fails at its next byte by itself. Larger tables use the same
+// two marks above their states.
+constexpr uint32_t kDead = 0xffu;
+__device__ __forceinline__ uint32_t next_byte(uint32_t next, uint32_t ns, uint32_t out) {
+  return next == kErr ? kDead : next < ns ? next : out;
 }
 
-template <bool LDS>
-__global__ __launch_bounds__(kThreads) void dfa_mask_kernel(const Params p) {
-  extern __shared__ __align__(16) uint32_t s_trans[];  // [num_states * 256] with LDS
-  const uint32_t tid = threadIdx.x, lane = tid & 63;
-  if (LDS) {
-    const uint32_t n4 = p.num_states * 64u;  // 16-byte groups
-    for (uint32_t i = tid; i < n4; i += kThreads) ((uint4*)s_trans)[i] = ((const uint4*)p.trans)[i];
+// How a block walks: kPerm8 every state of a table of up to 8, by composing
+// byte functions; kLds and kGlobal a list of up to 64 start states, one walk
+// per start state that accepts the token's first byte, through the table's
+// bytes in LDS or its words in memory.
+enum Walk { kPerm8, kLds, kGlobal };
+
+// Bytes [at, at + 16) of the token bytes, zeros past num_bytes. (Unaligned
+// 16-byte loads are one instruction.)
+struct __attribute__((packed)) Piece {
+  uint32_t w[4];
+};
+__device__ __forceinline__ void load_piece(const Params& p, uint32_t at, uint32_t (&w)[4]) {
+  if (p.num_bytes - at >= 16u) {  // (at <= num_bytes)
+    const Piece q = *(const Piece*)(p.bytes + at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = q.w[i];
+  } else {
+    uint64_t lo = 0, hi = 0;
+    for (uint32_t i = p.num_bytes - at; i-- > 0u;) {  // (at most 15)
+      hi = (hi << 8) | (lo >> 56);
+      lo = (lo << 8) | p.bytes[at + i];
+    }
+    w[0] = (uint32_t)lo;
+    w[1] = (uint32_t)(lo >> 32);
+    w[2] = (uint32_t)hi;
+    w[3] = (uint32_t)(hi >> 32);
+  }
+}
+
+// Masks of kTok * 256 tokens for a group of rows. by_state: the start states
+// are the table's own (num_states <= 64) and blockIdx.y picks kRows rows;
+// otherwise they are the states of the 64 rows that blockIdx.y picks.
+//
+// Measured, 128 rows x 128256 tokens, us per launch (in brackets: a walk of
+// every state per 32 rows or of every row per 16, byte loads and a ballot per
+// row): 8 states 7.3 (25.8), 16 states 16.9 (31.9), 64 states 32.8 (93.8), 69
+// states 41.6 (62.7), 154 states 30.5 (58.6); 8 rows, 64 states 9.7 (86.2).
+template <Walk WALK>
+__global__ __launch_bounds__(kThreads) void dfa_mask_kernel(const Params p, const uint32_t by_state) {
+  extern __shared__ __align__(16) uint8_t s_table[];  // kLds: [num_states][256] next states
+  __shared__ uint64_t s_fn[256];  // kPerm8: byte b's function; else: the start states that accept b
+  __shared__ uint32_t s_start[kList];
+  __shared__ uint32_t s_words[kList + 1][kWords];  // [start state][word]; the last: tokens with no bytes
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t ns = p.num_states;
+  const uint32_t out = WALK == kPerm8 ? 0x0du : 0xfeu;  // (kLds: num_states <= 128 < 0xfe)
+  const uint32_t words = (p.V + 31u) / 32u;
+  const uint32_t tbase = blockIdx.x * (kTok * kThreads);
+  const uint32_t r0 = blockIdx.y * (by_state ? (uint32_t)kRows : kList);
+  const uint32_t nr = min(by_state ? (uint32_t)kRows : kList, p.B - r0);
+  const uint32_t n_list = by_state ? ns : nr;
+
+  uint32_t b0[kTok], len[kTok], piece[kTok][4];
+  bool in[kTok];
+#pragma unroll
+  for (int k = 0; k < kTok; ++k) {
+    const uint32_t t = tbase + k * kThreads + tid;
+    in[k] = t < p.V;
+    const uint32_t at = in[k] ? t : 0u;
+    b0[k] = p.offsets[at];
+    const uint32_t e = p.offsets[at + 1];
+    if (e < b0[k] || e > p.num_bytes) in[k] = false;  // a range outside the byte array: not allowed, nothing read
+    len[k] = in[k] ? e - b0[k] : 0u;
+    if (!in[k]) b0[k] = 0u;
+  }
+  if (WALK != kPerm8) {
+    if (tid < kList) s_start[tid] = by_state ? tid : p.states[r0 + min(tid, nr - 1u)];
+    if (WALK == kLds)
+      for (uint32_t i = tid; i < ns * 64u; i += kThreads) {  // four entries per step
+        const uint32_t* q = p.trans + 4u * i;
+        uint32_t w = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w |= next_byte(q[e], ns, out) << (8 * e);
+        ((uint32_t*)s_table)[i] = w;
+      }
     __syncthreads();
   }
-  const uint32_t* T = LDS ? s_trans : p.trans;
-  const uint32_t ns = p.num_states;
-  const uint32_t r0 = blockIdx.y * kRowsPerBlock;
-  const uint32_t nr = min((uint32_t)kRowsPerBlock, p.B - r0);
-  const uint32_t words = (p.V + 31u) / 32u;
-  uint32_t st0[kRowsPerBlock];  // the row group's start states
 #pragma unroll
-  for (int q = 0; q < kRowsPerBlock; ++q) st0[q] = p.states[r0 + ((uint32_t)q < nr ? q : 0u)];
-  for (int k = 0; k < kTokPerThread; ++k) {
-    // consecutive tokens per wavefront, the wavefront's first one 64-aligned
-    const uint32_t t = (blockIdx.x * kTokPerThread + k) * kThreads + tid;
-    bool in = t < p.V;
-    uint32_t b0 = 0, len = 0;
-    if (in) {
-      b0 = p.offsets[t];
-      const uint32_t e = p.offsets[t + 1];
-      if (e >= b0 && e <= p.num_bytes) len = e - b0;
-      else in = false;  // a range outside the byte array: not allowed, nothing read
+  for (int k = 0; k < kTok; ++k)
+    if (len[k]) load_piece(p, b0[k], piece[k]);
+  {  // this thread's byte: its function, or the start states that accept it
+    uint64_t f = 0;
+    if constexpr (WALK == kPerm8) {
+      uint32_t nx[kPermStates];
+#pragma unroll
+      for (uint32_t s = 0; s < kPermStates; ++s) nx[s] = kErr;
+      if (ns) {
+#pragma unroll
+        for (uint32_t s = 0; s < kPermStates; ++s) nx[s] = p.trans[(s < ns ? s : 0u) * 256u + tid];
+      }
+#pragma unroll
+      for (uint32_t s = 0; s < kPermStates; ++s)
+        f |= (uint64_t)(s < ns ? next_byte(nx[s], ns, out) : kDead) << (8u * s);
+    } else {
+      for (uint32_t i0 = 0; i0 < n_list; i0 += 8u) {  // eight reads at a time
+        uint32_t nx[8], st[8];
+#pragma unroll
+        for (uint32_t e = 0; e < 8; ++e) {
+          st[e] = s_start[min(i0 + e, n_list - 1u)];
+          const uint32_t at = (st[e] < ns ? st[e] : 0u);
+          nx[e] = WALK == kLds ? (s_table[at * 256u + tid] == kDead ? kErr : 0u) : p.trans[(size_t)at * 256u + tid];
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < 8; ++e)
+          if (i0 + e < n_list && st[e] < ns && nx[e] != kErr) f |= 1ull << (i0 + e);
+      }
     }
-    uint32_t s[kRowsPerBlock];
-    bool ok[kRowsPerBlock];
+    s_fn[tid] = f;
+  }
+  __syncthreads();
+
 #pragma unroll
-    for (int q = 0; q < kRowsPerBlock; ++q) {
-      s[q] = st0[q];
-      ok[q] = in && (uint32_t)q < nr;
-    }
-    // the token's bytes kMaxBytes at a time, each piece read once and walked
-    // from every row's state (kRowIlp rows interleaved); a lane stops when no
-    // row can still allow its token
-    for (uint32_t j0 = 0; j0 < len; j0 += kMaxBytes) {
-      uint32_t by[kMaxBytes];
+  for (int k = 0; k < kTok; ++k) {
+    uint64_t alive = 0;  // bit i: the token walks from start state i
+    if constexpr (WALK == kPerm8) {
+      uint32_t lo = 0x03020100u, hi = 0x07060504u;  // the states reached, one byte each
+      for (uint32_t j0 = 0; j0 < len[k]; j0 += 16u) {
+        if (j0) load_piece(p, b0[k] + j0, piece[k]);
+        const uint32_t n = min(len[k] - j0, 16u);
 #pragma unroll
-      for (int j = 0; j < kMaxBytes; ++j) by[j] = j0 + j < len ? p.bytes[b0 + j0 + j] : 0u;
-      const uint32_t n = min(len - j0, (uint32_t)kMaxBytes);
-#pragma unroll
-      for (int q0 = 0; q0 < kRowsPerBlock; q0 += kRowIlp) {
-#pragma unroll
-        for (int j = 0; j < kMaxBytes; ++j) {
-          if ((uint32_t)j < n) {
-#pragma unroll
-            for (int q = q0; q < q0 + kRowIlp; ++q) step(T, ns, by[j], s[q], ok[q]);
+        for (uint32_t j = 0; j < 16; ++j) {
+          if (j < n) {
+            const uint64_t f = s_fn[(piece[k][j / 4] >> (8u * (j % 4u))) & 0xffu];
+            lo = __builtin_amdgcn_perm((uint32_t)(f >> 32), (uint32_t)f, lo);
+            hi = __builtin_amdgcn_perm((uint32_t)(f >> 32), (uint32_t)f, hi);
           }
         }
       }
-      bool any = false;
+      // (bytes below 0x80: a state, or kOut)
 #pragma unroll
-      for (int q = 0; q < kRowsPerBlock; ++q) any |= ok[q];
-      if (!any) break;
-    }
-    const uint32_t wbase = (t - lane) / 32u;  // the wavefront's first mask word
+      for (uint32_t s = 0; s < kPermStates; ++s)
+        alive |= (uint64_t)((~(s < 4u ? lo : hi) >> (8u * (s % 4u) + 7u)) & 1u) << s;
+      alive &= (1ull << ns) - 1ull;
+    } else if (len[k] == 0u) {
+      alive = ~0ull;
+    } else {
+      uint64_t todo = s_fn[piece[k][0] & 0xffu];
+      if (len[k] == 1u) {
+        alive = todo;
+      } else {
+        while (todo) {  // the start states that accept the first byte
+          const uint32_t i = (uint32_t)__builtin_ctzll(todo);
+          todo &= todo - 1u;
+          uint32_t c = s_start[i];
+          bool ok = true;
+          for (uint32_t j0 = 0; j0 < len[k] && ok; j0 += 16u) {
+            uint32_t w[4] = {piece[k][0], piece[k][1], piece[k][2], piece[k][3]};
+            if (j0) load_piece(p, b0[k] + j0, w);
+            const uint32_t n = min(len[k] - j0, 16u);
 #pragma unroll
-    for (int q = 0; q < kRowsPerBlock; ++q) {
-      const uint64_t m = __ballot(ok[q]);
-      if ((uint32_t)q < nr) {
-        uint32_t* row = p.mask + (size_t)(r0 + q) * p.mask_ld;
-        if (lane == 0 && wbase < words) row[wbase] = (uint32_t)m;
-        if (lane == 32 && wbase + 1 < words) row[wbase + 1] = (uint32_t)(m >> 32);
-      }
-    }
-  }
-}
-
-// Tables of at most 64 states: each token is walked once from every start
-// state at the same time (independent lookups), leaving a 64-bit word whose
-// bit s says whether the token walks from state s; each row's mask bit is then
-// one test of its own state's bit. That is num_states x length lookups per
-// token instead of rows x length. A state outside the table allows only tokens
-// with no bytes. A block covers kStTok * 256 tokens and kStRows rows; the mask
-// words of kStBatch rows at a time are gathered in LDS from the wavefronts'
-// ballots and written as one contiguous run per row.
-constexpr uint32_t kSetStates = 64;
-constexpr int kStTok = 2;     // tokens per thread
-constexpr int kStRows = 32;   // rows per block
-constexpr int kStBatch = 8;   // rows staged in LDS per round
-constexpr int kStWords = kStTok * kThreads / 32;  // mask words per row and block
-template <int NS, bool LDS>  // NS: a bound on num_states (8, 16 or 64)
-__global__ __launch_bounds__(kThreads) void dfa_mask_states_kernel(const Params p) {
-  extern __shared__ __align__(16) uint32_t s_trans[];  // [num_states * 256] with LDS
-  __shared__ uint32_t s_words[kStBatch][kStWords];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (LDS) {
-    const uint32_t n4 = p.num_states * 64u;
-    for (uint32_t i = tid; i < n4; i += kThreads) ((uint4*)s_trans)[i] = ((const uint4*)p.trans)[i];
-    __syncthreads();
-  }
-  const uint32_t* T = LDS ? s_trans : p.trans;
-  const uint32_t ns = p.num_states;  // <= NS
-  const uint32_t words = (p.V + 31u) / 32u;
-  const uint32_t tbase = blockIdx.x * (kStTok * kThreads);
-  const uint32_t r0 = blockIdx.y * kStRows;
-  const uint32_t nr = min((uint32_t)kStRows, p.B - r0);
-  const uint32_t my_state = p.states[r0 + (lane < nr ? lane : 0u)];  // lane q holds row r0 + q's state
-  uint64_t alive[kStTok];
-  bool empty[kStTok];
-#pragma unroll
-  for (int k = 0; k < kStTok; ++k) {
-    const uint32_t t = tbase + k * kThreads + tid;
-    bool in = t < p.V;
-    uint32_t b0 = 0, len = 0;
-    if (in) {
-      b0 = p.offsets[t];
-      const uint32_t e = p.offsets[t + 1];
-      if (e >= b0 && e <= p.num_bytes) len = e - b0;
-      else in = false;  // a range outside the byte array: not allowed, nothing read
-    }
-    uint32_t cur[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) cur[s] = (uint32_t)s;
-    uint64_t a = ns >= 64u ? ~0ull : ((1ull << ns) - 1ull);
-    if (!in) a = 0;
-    // the bytes kMaxBytes at a time, all loads of a piece issued together
-    for (uint32_t j0 = 0; j0 < len && a; j0 += kMaxBytes) {
-      uint32_t by[kMaxBytes];
-#pragma unroll
-      for (int j = 0; j < kMaxBytes; ++j) by[j] = j0 + j < len ? p.bytes[b0 + j0 + j] : 0u;
-      const uint32_t n = min(len - j0, (uint32_t)kMaxBytes);
-#pragma unroll
-      for (int j = 0; j < kMaxBytes; ++j) {
-        if ((uint32_t)j < n) {
-#pragma unroll
-          for (int s = 0; s < NS; ++s) {
-            if ((a >> s) & 1ull) {  // (DfaSchemaGrammar::transition, dfa.rs:110-126)
-              const uint32_t c = cur[s];
-              const uint32_t nxt = c < ns ? T[c * 256u + by[j]] : kErr;
-              if (nxt == kErr) a &= ~(1ull << s);
-              cur[s] = nxt;
+            for (uint32_t j = 0; j < 16; ++j) {
+              if (j < n && ok) {  // (DfaSchemaGrammar::transition, dfa.rs:110-126)
+                const uint32_t b = (w[j / 4] >> (8u * (j % 4u))) & 0xffu;
+                if (c >= ns) {
+                  ok = false;
+                } else if constexpr (WALK == kLds) {
+                  c = s_table[c * 256u + b];
+                  ok = c != kDead;
+                } else {
+                  c = p.trans[(size_t)c * 256u + b];
+                  ok = c != kErr;
+                }
+              }
             }
           }
+          if (ok) alive |= 1ull << i;
         }
       }
     }
-    alive[k] = a;
-    empty[k] = in && len == 0;  // allowed from every state, even outside the table
-  }
-  static_assert(kStRows <= 64, "one row state per lane");
-  for (uint32_t rb = 0; rb < nr; rb += kStBatch) {
-#pragma unroll
-    for (int q = 0; q < kStBatch; ++q) {
-      if (rb + q < nr) {
-        const uint32_t st = (uint32_t)__builtin_amdgcn_readlane((int)my_state, (int)(rb + q));
-#pragma unroll
-        for (int k = 0; k < kStTok; ++k) {
-          const bool ok = st < ns ? ((alive[k] >> st) & 1ull) != 0 : empty[k];
-          const uint64_t m = __ballot(ok);
-          const uint32_t w = (k * kThreads + 64u * wave) / 32u;  // block-local word of this ballot
-          if (lane == 0) {
-            s_words[q][w] = (uint32_t)m;
-            s_words[q][w + 1] = (uint32_t)(m >> 32);
-          }
-        }
-      }
+    if (!in[k]) alive = 0;
+    // lane i takes the ballot of start state i
+    const uint32_t w = (k * kThreads + 64u * wave) / 32u;
+    uint32_t mine_lo = 0, mine_hi = 0;
+    for (uint32_t i = 0; i < n_list; ++i) {
+      const uint64_t m = __ballot((alive >> i) & 1ull);
+      mine_lo = lane == i ? (uint32_t)m : mine_lo;
+      mine_hi = lane == i ? (uint32_t)(m >> 32) : mine_hi;
     }
-    __syncthreads();
-    if (tid < (uint32_t)(kStBatch * kStWords)) {
-      const uint32_t q = tid / kStWords, w = tid % kStWords;
-      const uint32_t gw = blockIdx.x * kStWords + w;
-      if (rb + q < nr && gw < words) p.mask[(size_t)(r0 + rb + q) * p.mask_ld + gw] = s_words[q][w];
+    if (lane < n_list) {
+      s_words[lane][w] = mine_lo;
+      s_words[lane][w + 1] = mine_hi;
     }
-    __syncthreads();
+    const uint64_t empty = __ballot(in[k] && len[k] == 0u);  // allowed from every state, even outside the table
+    if (lane == 0) {
+      s_words[kList][w] = (uint32_t)empty;
+      s_words[kList][w + 1] = (uint32_t)(empty >> 32);
+    }
   }
-}
-
-template <int NS>
-static void launch_states(const Params& p, dim3 grid, bool lds, size_t lds_bytes, hipStream_t st) {
-  if (lds) hipLaunchKernelGGL((dfa_mask_states_kernel<NS, true>), grid, dim3(kThreads), lds_bytes, st, p);
-  else hipLaunchKernelGGL((dfa_mask_states_kernel<NS, false>), grid, dim3(kThreads), 0, st, p);
+  __syncthreads();
+  for (uint32_t i = tid; i < nr * (uint32_t)kWords; i += kThreads) {
+    const uint32_t q = i / kWords, w = i % kWords;
+    const uint32_t gw = blockIdx.x * kWords + w;
+    uint32_t idx = q;
+    if (by_state) {
+      const uint32_t s = p.states[r0 + q];
+      idx = s < ns ? s : kList;
+    }
+    if (gw < words) p.mask[(size_t)(r0 + q) * p.mask_ld + gw] = s_words[idx][w];
+  }
 }
 
 // Row b of the output is row min(states[b], num_states) of the per-state
@@ -355,9 +378,8 @@ extern "C" int oxs_dfa_mask(const oxs_dfa* dfa, const oxs_token_bytes* tokens, c
   if ((dfa->num_states && !dfa->transitions) || !tokens->offsets || !tokens->bytes || !states || !mask)
     return OXS_ERR_INVALID_ARGUMENT;
   if (mask_ld < (int64_t)((tokens->vocab + 31u) / 32u)) return OXS_ERR_INVALID_ARGUMENT;
-  // token indices stay below 2^31 and row groups within the grid's y extent
-  if (tokens->vocab > (1u << 31) || batch > 65535u * (uint32_t)min(kRowsPerBlock, kStRows))
-    return OXS_ERR_INVALID_ARGUMENT;
+  // token indices stay below 2^31; the batch within 65535 groups of 16 rows
+  if (tokens->vocab > (1u << 31) || batch > 65535u * 16u) return OXS_ERR_INVALID_ARGUMENT;
   Params p;
   p.trans = dfa->transitions;
   p.num_states = dfa->num_states;
@@ -370,20 +392,16 @@ extern "C" int oxs_dfa_mask(const oxs_dfa* dfa, const oxs_token_bytes* tokens, c
   p.mask = mask;
   p.mask_ld = mask_ld;
   hipStream_t st = (hipStream_t)stream;
-  // the table is copied into LDS in 16-byte pieces: small and 16-byte aligned tables only
-  const bool lds = p.num_states <= kLdsStates && ((uintptr_t)p.trans & 15u) == 0;
-  const size_t lds_bytes = lds ? p.num_states * 256u * sizeof(uint32_t) : 0;
-  if (p.num_states <= kSetStates) {
-    const uint32_t per_block = (uint32_t)(kStTok * kThreads);
-    const dim3 grid((p.V + per_block - 1) / per_block, (batch + kStRows - 1) / kStRows);
-    if (p.num_states <= 8) launch_states<8>(p, grid, lds, lds_bytes, st);
-    else if (p.num_states <= 16) launch_states<16>(p, grid, lds, lds_bytes, st);
-    else launch_states<64>(p, grid, lds, lds_bytes, st);
-  } else {
-    const uint32_t per_block = (uint32_t)(kThreads * kTokPerThread);
-    const dim3 grid((p.V + per_block - 1) / per_block, (batch + kRowsPerBlock - 1) / kRowsPerBlock);
-    hipLaunchKernelGGL(dfa_mask_kernel<false>, grid, dim3(kThreads), 0, st, p);
-  }
+  const uint32_t ns = p.num_states;
+  // start states: the table's own when there are at most 64 and the rows are no
+  // fewer (or there are at most 8, which are walked at once), else the rows'
+  const uint32_t by_state = ns <= kPermStates || (ns <= kList && batch > ns) ? 1u : 0u;
+  const uint32_t per_block = (uint32_t)(kTok * kThreads), rows = by_state ? (uint32_t)kRows : kList;
+  const dim3 grid((p.V + per_block - 1) / per_block, (batch + rows - 1) / rows);
+  if (ns <= kPermStates) hipLaunchKernelGGL(dfa_mask_kernel<kPerm8>, grid, dim3(kThreads), 0, st, p, by_state);
+  else if (ns <= kLdsStates)
+    hipLaunchKernelGGL(dfa_mask_kernel<kLds>, grid, dim3(kThreads), ns * 256u, st, p, by_state);
+  else hipLaunchKernelGGL(dfa_mask_kernel<kGlobal>, grid, dim3(kThreads), 0, st, p, by_state);
   return hipGetLastError() == hipSuccess ? OXS_OK : OXS_ERR_HIP;
 }
 

@@ -172,6 +172,28 @@ def test_gpu_dfa_mask_matches_oracle(torch_gpu, n, V, B):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,V,B,density", [
+    (3, 511, 129, 0.5), (8, 513, 256, 0.9), (7, 512, 1, 0.9),        # whole functions, rows past one block's 128
+    (9, 512, 9, 0.5), (9, 513, 10, 0.5), (64, 1025, 65, 0.3),        # rows' states up to n rows, the table's above
+    (64, 31, 64, 1.0), (33, 4097, 200, 0.1), (128, 1000, 130, 0.4),  # the largest table in LDS
+    (129, 1000, 65, 0.4), (300, 33, 3, 0.6)])                        # and in memory
+def test_gpu_dfa_mask_walk_forms(torch_gpu, n, V, B, density):
+    # every form of the walk and its edges: tokens of 0 to 45 bytes, the vocabulary's last bytes,
+    # next states and row states outside the table
+    rng = np.random.default_rng(n * 31 + V + B)
+    table = random_dfa(rng, n, density)
+    vocab = random_vocab(rng, V, JSON_ALPHA + bytes(range(250, 256)), 20)
+    vocab[-1] = bytes(vocab[-1]) + b"{"  # ends at the last byte
+    states = rng.integers(0, n, size=B).astype(np.uint32)
+    states[B // 2] = n
+    states[-1] = ERR if B > 1 else 0
+    off, by = pack(vocab)
+    print(f"\n[case] dfa mask walk forms states={n} vocab={V} rows={B}", flush=True)
+    got = gpu_mask(torch_gpu, table, n, vocab, states)
+    np.testing.assert_array_equal(got, oracle.dfa_mask_host(table, n, off, by, states))
+
+
+@pytest.mark.gpu
 def test_gpu_dfa_mask_empty_table(torch_gpu):
     # no states: every state is outside the table, so only tokens with no bytes are allowed
     vocab = [b"", b"a", b"", b"{}", b"x" * 40]
