@@ -453,37 +453,49 @@ __device__ uint32_t block_excl_scan(uint32_t v, uint32_t* total, uint32_t* scrat
 // A stream block marks the sparse-stage ids of its chunk (history window
 // with counts, bans, biases, newline) in an open-addressing LDS hash keyed by
 // chunk offset.
-constexpr int kHashSlots = 256;
+//
+// The table takes as many slots as the row has sparse-stage ids, in steps of
+// 64 (a wavefront's visit), at least kHashMin and at most kHashSlots: it then holds every id of a row of up to 960 of
+// them, however skewed to one chunk. With 256 slots a window of 1024 ids, a
+// third of them in the vocabulary's first chunk, overflowed the table there,
+// and an overflow sends the whole row to the tail's exact re-scan: 256 rows of
+// 151936 bf16 logits took 2947 us, and take 57 with the table sized by the row
+// (64 rows x 128256, 512-id windows: 20.9 -> 18.9; one row x 32000, 64 ids: 12.8 -> 12.9,
+// the longer slot arithmetic).
+// 960 slots beside the 32 KB of staged values stay within a quarter of the
+// CU's 160 KB of LDS, so four blocks stay resident. Rows of up to 256 ids
+// visit 256 slots only; clearing all 960 is two 16-byte stores per thread
+// while the row's record is on its way.
+constexpr int kHashSlots = 960;
+constexpr int kHashMin = kThreads;  // a slot per thread
 constexpr uint32_t kEmptySlot = 0xffffffffu;
-__device__ __forceinline__ uint32_t hash_slot(uint32_t key) { return (key * 0x9e3779b1u) >> 24; }
-static_assert(kHashSlots == 256, "hash_slot yields 8 bits");
+static_assert(kHashSlots % 4 == 0 && kHashSlots / 4 <= kThreads, "cleared by one 16-byte store per thread");
+static_assert((kMaxChunk + 2 * kHashSlots) * 4 + 64 <= 160 * 1024 / 4, "four stream blocks per CU");
+__device__ __forceinline__ uint32_t hash_slots_of(const RowXf& r) {
+  const uint32_t most = (uint32_t)kHashSlots;
+  const uint32_t ids = (r.use_hist ? min(r.wn, most) : 0u) + min(r.ban_cnt, most) + min(r.bias_cnt, most) +
+                       (r.nl_active ? 1u : 0u);
+  return max((uint32_t)kHashMin, min((ids + 63u) & ~63u, most));
+}
+__device__ __forceinline__ uint32_t hash_slot(uint32_t key, uint32_t slots) {
+  return __umul24((key * 0x9e3779b1u) >> 16, slots) >> 16;  // (slots <= 2048)
+}
 
 // Continues an insertion whose home slot held another key; false when full.
-__device__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t key, uint32_t add, uint32_t orv) {
-  uint32_t h = hash_slot(key);
-  for (int probe = 0; probe < kHashSlots; ++probe) {
+__device__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t slots, uint32_t key, uint32_t add,
+                                 uint32_t orv) {
+  uint32_t h = hash_slot(key, slots);
+  for (uint32_t probe = 0; probe < slots; ++probe) {
     const uint32_t prev = atomicCAS(&hkeys[h], kEmptySlot, key);
     if (prev == kEmptySlot || prev == key) {
       if (add) atomicAdd(&hvals[h], add);
       if (orv) atomicOr(&hvals[h], orv);
       return true;
     }
-    h = (h + 1) & (kHashSlots - 1);
+    h = h + 1u == slots ? 0u : h + 1u;
   }
   return false;
 }
-
-__device__ __forceinline__ uint32_t hash_lookup(const uint32_t* hkeys, const uint32_t* hvals, uint32_t key) {
-  uint32_t h = hash_slot(key);
-  for (int probe = 0; probe < kHashSlots; ++probe) {
-    const uint32_t k = hkeys[h];
-    if (k == key) return hvals[h];
-    if (k == kEmptySlot) return 0u;
-    h = (h + 1) & (kHashSlots - 1);
-  }
-  return 0u;
-}
-
 
 // ---------------------------------------------------------------- stream kernel
 
@@ -503,7 +515,7 @@ template <int DT, int SLOTS, bool VEC, bool MASK, bool WB>
 __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint32_t chunk, const RowXf& r,
                                              const uint32_t (&raw)[SLOTS][kind_f32(DT) ? 4 : 8],
                                              const uint32_t (&mw)[SLOTS], float* s_x, uint32_t* s_hkeys,
-                                             uint32_t* s_hvals, uint32_t* s_full) {
+                                             uint32_t* s_hvals, uint32_t slots, uint32_t* s_full) {
   constexpr int EPL = kind_f32(DT) ? 4 : 8;
   constexpr int TILE = kThreads * EPL;
   constexpr int NE = SLOTS * EPL;
@@ -545,7 +557,7 @@ __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint
   // ---- sparse-stage ids at their exact values (sampler.rs:184-245)
   if (r.any_special) {
     __syncthreads();  // values staged, marks complete
-    for (uint32_t h = tid; h < (uint32_t)kHashSlots; h += kThreads) {
+    for (uint32_t h = tid; h < slots; h += kThreads) {
       const uint32_t off = s_hkeys[h];
       if (off != kEmptySlot) s_x[off] = apply_special(p.bias_ids, p.bias_values, r, s_x[off], s_hvals[h], c0 + off);
     }
@@ -649,7 +661,7 @@ __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint
 // with no barrier: the next block barrier completes the marks.
 __device__ __forceinline__ void build_marks(const Params& p, const RowXf& r, uint32_t row, uint32_t c0,
                                             uint32_t c1, const uint32_t (&hv)[kHistUnroll],
-                                            uint32_t* s_hkeys, uint32_t* s_hvals, uint32_t* s_full) {
+                                            uint32_t* s_hkeys, uint32_t* s_hvals, uint32_t slots, uint32_t* s_full) {
   const uint32_t tid = threadIdx.x;
   bool ok = true;
   uint32_t prev[kHistUnroll];
@@ -657,32 +669,32 @@ __device__ __forceinline__ void build_marks(const Params& p, const RowXf& r, uin
   for (int q = 0; q < kHistUnroll; ++q) {
     const uint32_t t = r.use_hist && tid + q * kThreads < r.wn ? hv[q] : 0xffffffffu;
     const bool in = t >= c0 && t < c1;
-    prev[q] = in ? atomicCAS(&s_hkeys[hash_slot(t - c0)], kEmptySlot, t - c0) : 0u;
+    prev[q] = in ? atomicCAS(&s_hkeys[hash_slot(t - c0, slots)], kEmptySlot, t - c0) : 0u;
   }
 #pragma unroll
   for (int q = 0; q < kHistUnroll; ++q) {
     const uint32_t t = r.use_hist && tid + q * kThreads < r.wn ? hv[q] : 0xffffffffu;
     if (!(t >= c0 && t < c1)) continue;
-    if (prev[q] == kEmptySlot || prev[q] == t - c0) atomicAdd(&s_hvals[hash_slot(t - c0)], 1u);
-    else ok &= hash_insert_from(s_hkeys, s_hvals, t - c0, 1u, 0u);
+    if (prev[q] == kEmptySlot || prev[q] == t - c0) atomicAdd(&s_hvals[hash_slot(t - c0, slots)], 1u);
+    else ok &= hash_insert_from(s_hkeys, s_hvals, slots, t - c0, 1u, 0u);
   }
   if (r.use_hist) {
     const uint32_t* hrow = p.history + (size_t)row * p.history_ld + r.wstart;
     for (uint32_t j = tid + kHistUnroll * kThreads; j < r.wn; j += kThreads) {  // long windows
       const uint32_t t = hrow[j];
-      if (t >= c0 && t < c1) ok &= hash_insert_from(s_hkeys, s_hvals, t - c0, 1u, 0u);
+      if (t >= c0 && t < c1) ok &= hash_insert_from(s_hkeys, s_hvals, slots, t - c0, 1u, 0u);
     }
   }
   for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
     const uint32_t id = p.ban_ids[r.ban_off + k];
-    if (id >= c0 && id < c1) ok &= hash_insert_from(s_hkeys, s_hvals, id - c0, 0u, kBanFlag);
+    if (id >= c0 && id < c1) ok &= hash_insert_from(s_hkeys, s_hvals, slots, id - c0, 0u, kBanFlag);
   }
   for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
     const uint32_t id = p.bias_ids[r.bias_off + k];
-    if (id >= c0 && id < c1) ok &= hash_insert_from(s_hkeys, s_hvals, id - c0, 0u, kBiasFlag);
+    if (id >= c0 && id < c1) ok &= hash_insert_from(s_hkeys, s_hvals, slots, id - c0, 0u, kBiasFlag);
   }
   if (tid == 0 && r.nl_active && r.nl_id >= c0 && r.nl_id < c1)
-    ok &= hash_insert_from(s_hkeys, s_hvals, r.nl_id - c0, 0u, kNlFlag);
+    ok &= hash_insert_from(s_hkeys, s_hvals, slots, r.nl_id - c0, 0u, kNlFlag);
   if (!ok) *s_full = 1;
 }
 
@@ -712,8 +724,8 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
   static_assert(NE <= 32, "one survivor bit per logit of a lane");
 
   __shared__ __align__(16) float s_x[NE * kThreads];  // each thread's masked raw logits (private slots)
-  __shared__ uint32_t s_hkeys[kHashSlots];
-  __shared__ uint32_t s_hvals[kHashSlots];
+  __shared__ __align__(16) uint32_t s_hkeys[kHashSlots];
+  __shared__ __align__(16) uint32_t s_hvals[kHashSlots];
   __shared__ uint32_t s_full;
 
   const uint32_t tid = threadIdx.x;
@@ -770,9 +782,9 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
       mw[s] = p.mask[(size_t)row * p.mask_ld + ((b2 < c1 ? b2 : p.V - 1) >> 5)];
     }
   }
-  for (uint32_t i = tid; i < (uint32_t)kHashSlots; i += kThreads) {
-    s_hkeys[i] = kEmptySlot;
-    s_hvals[i] = 0;
+  if (tid < (uint32_t)kHashSlots / 4u) {
+    *(uint4*)&s_hkeys[4 * tid] = make_uint4(kEmptySlot, kEmptySlot, kEmptySlot, kEmptySlot);
+    *(uint4*)&s_hvals[4 * tid] = make_uint4(0u, 0u, 0u, 0u);
   }
   if (tid == 0) s_full = 0;
   __builtin_amdgcn_sched_barrier(0);
@@ -786,6 +798,7 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
   const uint32_t hlen = (uint32_t)__builtin_amdgcn_readlane((int)rec, 26);
   if ((kflags & kKDecode) && cfg.temperature <= 1e-6f) raw_argmax_config(cfg);  // continuous_batching.rs:961
   const RowXf r = make_row_xf(cfg, hlen, V, history_ld, kflags);
+  const uint32_t slots = hash_slots_of(r);
   // history window ids, read without a branch (an in-bounds dummy address
   // where the row has none)
   uint32_t hv[kHistUnroll];
@@ -810,10 +823,10 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
   }
   if (r.any_special) {
     __syncthreads();  // tables cleared
-    build_marks(p, r, row, c0, c1, hv, s_hkeys, s_hvals, &s_full);
+    build_marks(p, r, row, c0, c1, hv, s_hkeys, s_hvals, slots, &s_full);
   }
 
-  process_unit<DT, SLOTS, VEC, MASK, WB>(p, row, chunk, r, raw, mw, s_x, s_hkeys, s_hvals, &s_full);
+  process_unit<DT, SLOTS, VEC, MASK, WB>(p, row, chunk, r, raw, mw, s_x, s_hkeys, s_hvals, slots, &s_full);
 }
 
 // ---------------------------------------------------------------- tail helpers
