@@ -460,8 +460,9 @@ __device__ uint32_t block_excl_scan(uint32_t v, uint32_t* total, uint32_t* scrat
 // third of them in the vocabulary's first chunk, overflowed the table there,
 // and an overflow sends the whole row to the tail's exact re-scan: 256 rows of
 // 151936 bf16 logits took 2947 us, and take 57 with the table sized by the row
-// (64 rows x 128256, 512-id windows: 20.9 -> 18.9; one row x 32000, 64 ids: 12.8 -> 12.9,
-// the longer slot arithmetic).
+// (64 rows x 128256, 512-id windows: 20.9 -> 18.9; one row x 32000, 64 ids: 12.8 -> 12.9 or
+// 13.0 -> 13.0; 512 rows x 262144, 257-id windows: 94.0 -> 95.6 or 94.5 -> 95.1, a
+// fifth wavefront visit and the longer slot arithmetic).
 // 960 slots beside the 32 KB of staged values stay within a quarter of the
 // CU's 160 KB of LDS, so four blocks stay resident. Rows of up to 256 ids
 // visit 256 slots only; clearing all 960 is two 16-byte stores per thread
@@ -1062,6 +1063,142 @@ __device__ __forceinline__ uint32_t exact_select_row(const Params& p, const RowX
     __syncthreads();
   }
   return meff;
+}
+
+// The row's top M where the candidate keys alone do not prove it: a pool of
+// more than 256 keys (top_k > 256), or a wavefront whose list or whose chunk's
+// hash overflowed. The stream kernel's records still bound the M-th key from
+// below: with t the largest threshold such that the wavefronts at or above it
+// emitted M keys, M keys have an order key of t - 1 or more (an emitted key may
+// lie one below its wavefront's recorded threshold, which is past the scaled
+// value that unemitted keys can reach). A wavefront whose threshold is at most
+// t - 1 emitted every such key; only the others' logits are read again, once,
+// compared with t - 1 before any mask or penalty is looked at. Ids with
+// sparse stages are skipped there and evaluated exactly from one hash of the
+// row's ids. What is found is sorted; its first M keys are the row's.
+//
+// Bound: latency of one block's reads (16 per lane in flight) and the sort. The
+// radix select below reads the whole row five times or more and rebuilds its
+// penalty table per chunk and pass: 16 rows x 128256, top_k 1000, 512-id
+// windows took 787 to 835 us a call with it and take 192 with this.
+//
+// Returns M, with the keys sorted in area[kRecHash ...], or 0 where this does
+// not apply and nothing was written: DRY rows (their candidates predate DRY),
+// a write-back (the radix select repairs it), more ids than the hash takes,
+// thresholds that bound too few keys (few wavefronts and a large M), more keys
+// than fit. area: kTailArea words; rec: 3 * kThreads words.
+constexpr int kRecHash = 2048;  // row-wide slots of sparse-stage ids (a key and an entry each)
+constexpr int kRecIds = 1536;   // ids at most
+constexpr int kRecCands = 2048;
+static_assert(kRecHash + kRecCands <= kTailArea && kMaxM <= kRecCands, "record selection fits the key area");
+static_assert(kMaxChunks * kWavesPerBlock <= kThreads, "a thread per wavefront record");
+template <int DT>
+__device__ __forceinline__ uint32_t record_select_row(const Params& p, const RowXf& r, uint32_t row, uint32_t M,
+                                                      uint64_t* area, uint32_t* rec, TailShared& ts) {
+  constexpr uint32_t EPL = kind_f32(DT) ? 4 : 8, RUN = 64 * EPL, TILE = kThreads * EPL;
+  constexpr int U = 16;  // logits per lane in flight
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t W = p.S * kWavesPerBlock, most = (uint32_t)kRecIds + 1u;
+  const uint32_t ids = (r.use_hist ? min(r.wn, most) : 0u) + min(r.ban_cnt, most) + min(r.bias_cnt, most) +
+                       (r.nl_active ? 1u : 0u);
+  if (r.dry || p.logits_out || ids > (uint32_t)kRecIds) return 0;
+  uint32_t *s_th = rec, *s_cnt = rec + kThreads, *s_need = rec + 2 * kThreads;
+  uint32_t *hk = (uint32_t*)area, *hv = hk + kRecHash;
+  uint64_t* cand = area + kRecHash;
+  __syncthreads();  // the block is done with area and rec
+  uint32_t th = ~0u, cnt = 0;  // (a bad record's values)
+  if (tid < W) {
+    th = (uint32_t)(p.wave_theta[(size_t)row * W + tid] >> 32);
+    cnt = p.wave_count[(size_t)row * W + tid];
+  }
+  s_th[tid] = th;
+  s_cnt[tid] = cnt;
+  for (uint32_t h = tid; h < (uint32_t)kRecHash; h += kThreads) {
+    hk[h] = kEmptySlot;
+    hv[h] = 0;
+  }
+  if (tid == 0) {
+    ts.counter = 0;
+    ts.sel_digit = 0;
+  }
+  __syncthreads();
+  uint32_t emitted = 0;
+  for (uint32_t j = 0; j < W; ++j) emitted += s_th[j] >= th ? s_cnt[j] : 0u;
+  if (th != ~0u && emitted >= M) atomicMax(&ts.sel_digit, th);
+  __syncthreads();
+  const uint32_t t = ts.sel_digit;
+  if (t == 0u) return 0;
+  const uint32_t T = t - 1u;
+  s_need[tid] = tid < W && th > T ? 1u : 0u;
+  if (r.use_hist) {
+    const uint32_t* win = p.history + (size_t)row * p.history_ld + r.wstart;
+    for (uint32_t j = tid; j < r.wn; j += kThreads)
+      if (win[j] < p.V) hash_insert_from(hk, hv, kRecHash, win[j], 1u, 0u);
+  }
+  for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
+    const uint32_t id = p.ban_ids[r.ban_off + k];
+    if (id < p.V) hash_insert_from(hk, hv, kRecHash, id, 0u, kBanFlag);
+  }
+  for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
+    const uint32_t id = p.bias_ids[r.bias_off + k];
+    if (id < p.V) hash_insert_from(hk, hv, kRecHash, id, 0u, kBiasFlag);
+  }
+  if (tid == 0 && r.nl_active) hash_insert_from(hk, hv, kRecHash, r.nl_id, 0u, kNlFlag);
+  __syncthreads();
+  const auto push = [&](uint64_t key) {
+    const uint32_t q = atomicAdd(&ts.counter, 1u);
+    if (q < (uint32_t)kRecCands) cand[q] = key;
+  };
+  const auto special = [&](uint32_t id) {
+    for (uint32_t h = hash_slot(id, kRecHash); hk[h] != kEmptySlot; h = (h + 1u) & (kRecHash - 1u))
+      if (hk[h] == id) return true;
+    return false;
+  };
+  const uint64_t* list = p.lists + (size_t)row * W * p.cap_w;
+  for (uint32_t i = tid; i < W * p.cap_w; i += kThreads) {
+    const uint32_t w = i >> p.cap_shift;
+    if (s_need[w] || (i & (p.cap_w - 1u)) >= s_cnt[w]) continue;
+    const uint64_t key = list[i];
+    if ((uint32_t)(key >> 32) >= T) push(key);
+  }
+  for (uint32_t w = wave; w < W; w += kWavesPerBlock) {
+    if (!s_need[w]) continue;
+    const uint32_t c0 = (w / kWavesPerBlock) * p.CH, c1 = min(c0 + p.CH, p.V);
+    const uint32_t first = c0 + (w % kWavesPerBlock) * RUN + lane;  // a wavefront holds RUN logits of every tile
+    for (uint32_t g0 = 0; g0 * 64u < p.CH / kWavesPerBlock; g0 += U) {
+      float x[U];
+#pragma unroll
+      for (uint32_t u = 0; u < (uint32_t)U; ++u) {
+        const uint32_t idx = first + ((g0 + u) / EPL) * TILE + ((g0 + u) % EPL) * 64u;
+        x[u] = load_logit<DT>(p, row, idx < c1 ? idx : c0);
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < (uint32_t)U; ++u) {
+        const uint32_t idx = first + ((g0 + u) / EPL) * TILE + ((g0 + u) % EPL) * 64u;
+        const uint32_t k = cand_key(r.do_temp ? x[u] * r.inv_temp : x[u]);
+        if (idx >= c1 || k == 0u || k < T) continue;
+        if (p.mask && !mask_allows(p, row, idx)) continue;
+        if (r.any_special && special(idx)) continue;
+        push(comp_key(k, idx));
+      }
+    }
+  }
+  for (uint32_t h = tid; h < (uint32_t)kRecHash; h += kThreads) {
+    const uint32_t id = hk[h];
+    if (id == kEmptySlot) continue;
+    const uint32_t chunk = id / p.CH, off = id - chunk * p.CH;
+    if (!s_need[chunk * kWavesPerBlock + (off % TILE) / RUN]) continue;
+    float x = load_logit<DT>(p, row, id);
+    if (p.mask && !mask_allows(p, row, id)) x = neg_inf();
+    x = apply_special(p.bias_ids, p.bias_values, r, x, hv[h], id);
+    const uint32_t k = cand_key(r.do_temp ? x * r.inv_temp : x);
+    if (k != 0u && k >= T) push(comp_key(k, id));
+  }
+  __syncthreads();
+  const uint32_t N = ts.counter;
+  if (N < M || N > (uint32_t)kRecCands) return 0;
+  bitonic_sort<false>(cand, N);
+  return M;
 }
 
 __device__ __forceinline__ float key_value(uint64_t k) { return ord2f((uint32_t)(k >> 32)); }

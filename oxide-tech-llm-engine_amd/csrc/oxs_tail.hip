@@ -7,7 +7,9 @@
 
 namespace oxs {
 
-template <int DT, int PER>
+// REC: rows whose candidates do not prove their top M try the wavefront
+// records before the radix select.
+template <int DT, int PER, bool REC>
 // Leading arguments: what the first loads need, preloaded into SGPRs as in
 // stream_kernel.
 __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restrict__ wave_theta,
@@ -27,6 +29,7 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
   __shared__ __align__(16) uint32_t s_bstart_all[kWavesPerBlock][kBuckets];  // one copy per wavefront
   __shared__ TailShared ts;
   __shared__ LibmTables s_tab;
+  static_assert(sizeof(s_bstart_all) >= 3 * kThreads * sizeof(uint32_t), "record selection's tables");
   static_assert(sizeof(uint32_t) * kChainLd * 3 + sizeof(uint64_t) * kChainLd <= sizeof(s_keys),
                 "chain scratch fits the key area");
 
@@ -311,13 +314,22 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
     }
   }
   if (path == 2) {
-    meff = exact_select_row<DT>(p, r, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
-    if (meff == 0) {
-      write_row_result<DT>(p, row, 0u, OXS_ROW_EMPTY, rs);
-      return;
+    const uint64_t* top = s_keys + kRecHash;
+    meff = 0;
+    if constexpr (REC) {
+      meff = record_select_row<DT>(p, r, row, M, s_keys, &s_bstart_all[0][0], ts);
+      __syncthreads();  // (every wavefront has read what the attempt left in LDS)
     }
-    bitonic_sort<false>(s_top, meff);
-    keys_to_chain(s_top, meff, s_ids, s_pr, s_tab);
+    if (meff == 0) {
+      meff = exact_select_row<DT>(p, r, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
+      if (meff == 0) {
+        write_row_result<DT>(p, row, 0u, OXS_ROW_EMPTY, rs);
+        return;
+      }
+      bitonic_sort<false>(s_top, meff);
+      top = s_top;
+    }
+    keys_to_chain(top, meff, s_ids, s_pr, s_tab);
   }
 
   // 5. the chain after the top-M selection, in the first wavefront
@@ -406,17 +418,32 @@ __global__ __launch_bounds__(kThreads) void wide_kernel(const Params p) {
   wave_chain<DT>(p, c, row, meff, bf, rs, s_tab);
 }
 
-template <int KIND>
-static hipError_t launch_tail_k(const Params& p, uint32_t grid_b, hipStream_t st) {
+template <int KIND, bool REC>
+static void launch_tail_rec(const Params& p, uint32_t grid_b, hipStream_t st) {
   // the row's candidate union: 2048 keys, or 4096 past 64 wavefront records
   if ((uint64_t)p.S * kWavesPerBlock * p.cap_w > (uint64_t)kUnionMax)
-    hipLaunchKernelGGL((tail_kernel<KIND, kUnionBig / kThreads>), dim3(grid_b), dim3(kThreads), 0, st,
+    hipLaunchKernelGGL((tail_kernel<KIND, kUnionBig / kThreads, REC>), dim3(grid_b), dim3(kThreads), 0, st,
                        (const uint64_t*)p.wave_theta, (const uint64_t*)p.lists, (const uint32_t*)p.wave_count, p.libm,
                        p.S, p.cap_w, p.cap_shift, p.rpx, p.B, p);
   else
-    hipLaunchKernelGGL((tail_kernel<KIND, kPer>), dim3(grid_b), dim3(kThreads), 0, st, (const uint64_t*)p.wave_theta,
-                       (const uint64_t*)p.lists, (const uint32_t*)p.wave_count, p.libm, p.S, p.cap_w, p.cap_shift,
-                       p.rpx, p.B, p);
+    hipLaunchKernelGGL((tail_kernel<KIND, kPer, REC>), dim3(grid_b), dim3(kThreads), 0, st,
+                       (const uint64_t*)p.wave_theta, (const uint64_t*)p.lists, (const uint32_t*)p.wave_count, p.libm,
+                       p.S, p.cap_w, p.cap_shift, p.rpx, p.B, p);
+}
+
+// The record selection is compiled into the tail only where the sampler was
+// created for pools above 256 (max_top_k > 256): those rows need it on nearly
+// every call, while its mere presence costs every row 0.4 us (one row x 32000:
+// 12.9 -> 13.3, 24 x 50257: 17.0 -> 17.4), and rows of 256 keys rarely leave the
+// candidate path. Softcap and decode-step kinds keep the radix select alone.
+template <int KIND>
+static hipError_t launch_tail_k(const Params& p, uint32_t grid_b, hipStream_t st) {
+  if constexpr (!kind_softcap(KIND) && !kind_decode(KIND)) {
+    if (p.wide_cap > 256u) launch_tail_rec<KIND, true>(p, grid_b, st);
+    else launch_tail_rec<KIND, false>(p, grid_b, st);
+  } else {
+    launch_tail_rec<KIND, false>(p, grid_b, st);
+  }
   if (p.wide_keys) hipLaunchKernelGGL((wide_kernel<KIND>), dim3(p.B), dim3(kThreads), 0, st, p);
   return hipGetLastError();
 }

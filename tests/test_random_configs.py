@@ -159,6 +159,65 @@ def test_logits_out_when_penalty_ids_overflow_the_chunk_hash(torch_gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [255, 256, 257, 320, 321, 960, 961, 1024])
+def test_penalty_ids_at_the_sizes_of_the_chunk_hash(torch_gpu, n):
+    # n distinct window ids in one stream chunk: the hash takes 256 slots, then steps of 64 up to
+    # 960, exactly full at 256, 320 and 960; from 961 on it overflows and the row is re-scanned
+    rng = np.random.default_rng(n)
+    B, V = 3, 1024
+    logits = (rng.standard_normal((B, V)) * 2.0).astype(np.float32)
+    history = np.stack([rng.permutation(V)[:n].astype(np.uint32) for _ in range(B)])
+    configs = [wl.disabled_config(frequency_penalty=0.6, presence_penalty=0.2, repeat_last_n=0),
+               wl.disabled_config(repeat_penalty=1.3, repeat_last_n=0, temperature=0.7),
+               wl.disabled_config(presence_penalty=-0.2, top_k=300, top_p=0.9, repeat_last_n=0)]
+    w = wl.Workload(name=f"{n} penalty ids in a chunk", logits=logits, dtype="f32", configs=configs,
+                    history=history, history_len=np.full(B, n, np.uint32), uniforms=wl.xorshift_uniforms(B, n))
+    banner(w.name)
+    for out in (True, False):
+        g = run_gpu(w, torch_gpu, logits_out=out, record=False, max_top_k=300)
+        r = run_oracle(w, logits_out=out, record=False)
+        compare(g, r, RTOL_F32, w.name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,vocab,dtype,kind", [
+    (3, 16384, "f32", "topk"), (3, 50257, "f32", "topk"), (3, 128256, "bf16", "topk"), (64, 151936, "bf16", "topk"),
+    (3, 50257, "f32", "ties"), (3, 128256, "bf16", "ties"), (3, 128256, "f32", "nan"), (2, 300001, "f32", "topk")])
+def test_top_m_from_the_wavefront_records(torch_gpu, batch, vocab, dtype, kind):
+    # rows whose candidate lists do not prove their top M, so that the wavefronts' thresholds bound it and
+    # part of the row is read again: pools of 257 to 1024 keys; runs of equal values that overflow some
+    # lists; NaN and infinities. Masks, biases, bans and window ids among the values read again.
+    rng = np.random.default_rng(batch * 1000003 + vocab)
+    x = (rng.standard_normal((batch, vocab)) * 3.0).astype(np.float32)
+    if kind == "ties":
+        x[:, 2048:2048 + 400] = 7.0
+        x[:, vocab - 300:] = 7.0
+    if kind == "nan":
+        x[:, 100:6000] = np.nan
+        x[0, 7000], x[1, 9000:9500] = np.inf, -np.inf
+    if dtype == "bf16":
+        x = (x.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    hist = (rng.random((batch, 700)) ** 3 * vocab).astype(np.uint32)
+    hist[:, :40] = np.argsort(-np.nan_to_num(x, nan=-9.0), axis=1)[:, :40]  # penalised ids among the largest
+    configs = []
+    for i in range(batch):
+        c = wl.disabled_config(repeat_penalty=1.2, frequency_penalty=-0.3, repeat_last_n=0, temperature=0.8,
+                               top_k=[257, 1000, 1024][i % 3] if kind == "topk" else 256, top_p=0.99)
+        c.logit_biases = {int(j): float(v) for j, v in zip(rng.integers(0, vocab, 40), rng.uniform(-4, 12, 40))}
+        c.banned_tokens = {int(j) for j in hist[i, :5]}
+        configs.append(c)
+    mask = rng.integers(0, 2**32, size=(batch, (vocab + 31) // 32), dtype=np.uint32) if vocab != 50257 else None
+    logits = (x.view(np.uint32) >> 16).astype(np.uint16) if dtype == "bf16" else x
+    w = wl.Workload(name=f"{kind} {batch} x {vocab} {dtype}", logits=logits, dtype=dtype, configs=configs,
+                    history=hist, history_len=np.full(batch, 700, np.uint32), mask=mask,
+                    uniforms=wl.xorshift_uniforms(batch, vocab))
+    banner(w.name)
+    g = run_gpu(w, torch_gpu, kept_ld=1024, record=False, max_top_k=1024)
+    r = run_oracle(w, kept_ld=1024, record=False, n_threads=8)
+    compare(g, r, RTOL_BF16 if dtype == "bf16" else RTOL_F32, w.name)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("seed", range(5000, 5008))
 def test_random_decode_steps(torch_gpu, seed):
     # oxs_decode_step over three steps with random configs (raw-argmax rows included) and
