@@ -469,24 +469,29 @@ __device__ uint32_t block_excl_scan(uint32_t v, uint32_t* total, uint32_t* scrat
 // while the row's record is on its way.
 constexpr int kHashSlots = 960;
 constexpr int kHashMin = kThreads;  // a slot per thread
+constexpr uint32_t kHashProbes = 128;  // slots an insertion of a row with more ids than the table looks at
 constexpr uint32_t kEmptySlot = 0xffffffffu;
 static_assert(kHashSlots % 4 == 0 && kHashSlots / 4 <= kThreads, "cleared by one 16-byte store per thread");
 static_assert((kMaxChunk + 2 * kHashSlots) * 4 + 64 <= 160 * 1024 / 4, "four stream blocks per CU");
-__device__ __forceinline__ uint32_t hash_slots_of(const RowXf& r) {
-  const uint32_t most = (uint32_t)kHashSlots;
-  const uint32_t ids = (r.use_hist ? min(r.wn, most) : 0u) + min(r.ban_cnt, most) + min(r.bias_cnt, most) +
-                       (r.nl_active ? 1u : 0u);
-  return max((uint32_t)kHashMin, min((ids + 63u) & ~63u, most));
+// The row's sparse-stage ids, counted up to one more than the hash takes.
+__device__ __forceinline__ uint32_t hash_ids_of(const RowXf& r) {
+  const uint32_t most = (uint32_t)kHashSlots + 1u;
+  return min((r.use_hist ? min(r.wn, most) : 0u) + min(r.ban_cnt, most) + min(r.bias_cnt, most) +
+                 (r.nl_active ? 1u : 0u),
+             most);
+}
+__device__ __forceinline__ uint32_t hash_slots_of(uint32_t ids) {
+  return max((uint32_t)kHashMin, min((ids + 63u) & ~63u, (uint32_t)kHashSlots));
 }
 __device__ __forceinline__ uint32_t hash_slot(uint32_t key, uint32_t slots) {
   return __umul24((key * 0x9e3779b1u) >> 16, slots) >> 16;  // (slots <= 2048)
 }
 
-// Continues an insertion whose home slot held another key; false when full.
-__device__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t slots, uint32_t key, uint32_t add,
-                                 uint32_t orv) {
+// Continues an insertion whose home slot held another key; false when `probes` slots held others.
+__device__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t slots, uint32_t probes, uint32_t key,
+                                 uint32_t add, uint32_t orv) {
   uint32_t h = hash_slot(key, slots);
-  for (uint32_t probe = 0; probe < slots; ++probe) {
+  for (uint32_t probe = 0; probe < probes; ++probe) {
     const uint32_t prev = atomicCAS(&hkeys[h], kEmptySlot, key);
     if (prev == kEmptySlot || prev == key) {
       if (add) atomicAdd(&hvals[h], add);
@@ -660,11 +665,22 @@ __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint
 // history window occurrence, a flag per ban, bias and newline. The first claim
 // of every window id's home slot goes out at once, collisions after. Ends
 // with no barrier: the next block barrier completes the marks.
+//
+// A row with more ids than the table takes may fill it. Its insertions give up
+// after kHashProbes slots (the table is then full, or so nearly that the row
+// goes to the exact re-scan anyway), and nothing more is inserted once one has
+// given up. 64 rows x 128256: windows of 30000 distinct ids 2257 us (13064 with
+// every failing insertion looking at all 960 slots), of 1000 in 1024 733 (991).
 __device__ __forceinline__ void build_marks(const Params& p, const RowXf& r, uint32_t row, uint32_t c0,
                                             uint32_t c1, const uint32_t (&hv)[kHistUnroll],
-                                            uint32_t* s_hkeys, uint32_t* s_hvals, uint32_t slots, uint32_t* s_full) {
+                                            uint32_t* s_hkeys, uint32_t* s_hvals, uint32_t slots, bool many, uint32_t* s_full) {
   const uint32_t tid = threadIdx.x;
-  bool ok = true;
+  const uint32_t probes = many ? kHashProbes : slots;
+  volatile uint32_t* full = s_full;
+  const auto insert = [&](uint32_t key, uint32_t add, uint32_t orv) {
+    if (many && *full) return;
+    if (!hash_insert_from(s_hkeys, s_hvals, slots, probes, key, add, orv)) *full = 1;
+  };
   uint32_t prev[kHistUnroll];
 #pragma unroll
   for (int q = 0; q < kHistUnroll; ++q) {
@@ -677,26 +693,26 @@ __device__ __forceinline__ void build_marks(const Params& p, const RowXf& r, uin
     const uint32_t t = r.use_hist && tid + q * kThreads < r.wn ? hv[q] : 0xffffffffu;
     if (!(t >= c0 && t < c1)) continue;
     if (prev[q] == kEmptySlot || prev[q] == t - c0) atomicAdd(&s_hvals[hash_slot(t - c0, slots)], 1u);
-    else ok &= hash_insert_from(s_hkeys, s_hvals, slots, t - c0, 1u, 0u);
+    else insert(t - c0, 1u, 0u);
   }
   if (r.use_hist) {
     const uint32_t* hrow = p.history + (size_t)row * p.history_ld + r.wstart;
     for (uint32_t j = tid + kHistUnroll * kThreads; j < r.wn; j += kThreads) {  // long windows
+      if (many && *full) break;
       const uint32_t t = hrow[j];
-      if (t >= c0 && t < c1) ok &= hash_insert_from(s_hkeys, s_hvals, slots, t - c0, 1u, 0u);
+      if (t >= c0 && t < c1) insert(t - c0, 1u, 0u);
     }
   }
   for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
     const uint32_t id = p.ban_ids[r.ban_off + k];
-    if (id >= c0 && id < c1) ok &= hash_insert_from(s_hkeys, s_hvals, slots, id - c0, 0u, kBanFlag);
+    if (id >= c0 && id < c1) insert(id - c0, 0u, kBanFlag);
   }
   for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
     const uint32_t id = p.bias_ids[r.bias_off + k];
-    if (id >= c0 && id < c1) ok &= hash_insert_from(s_hkeys, s_hvals, slots, id - c0, 0u, kBiasFlag);
+    if (id >= c0 && id < c1) insert(id - c0, 0u, kBiasFlag);
   }
   if (tid == 0 && r.nl_active && r.nl_id >= c0 && r.nl_id < c1)
-    ok &= hash_insert_from(s_hkeys, s_hvals, slots, r.nl_id - c0, 0u, kNlFlag);
-  if (!ok) *s_full = 1;
+    insert(r.nl_id - c0, 0u, kNlFlag);
 }
 
 // One (row, chunk) per block. The first half of the chunk's logits is issued
@@ -799,7 +815,7 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
   const uint32_t hlen = (uint32_t)__builtin_amdgcn_readlane((int)rec, 26);
   if ((kflags & kKDecode) && cfg.temperature <= 1e-6f) raw_argmax_config(cfg);  // continuous_batching.rs:961
   const RowXf r = make_row_xf(cfg, hlen, V, history_ld, kflags);
-  const uint32_t slots = hash_slots_of(r);
+  const uint32_t ids = hash_ids_of(r), slots = hash_slots_of(ids);
   // history window ids, read without a branch (an in-bounds dummy address
   // where the row has none)
   uint32_t hv[kHistUnroll];
@@ -824,7 +840,7 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
   }
   if (r.any_special) {
     __syncthreads();  // tables cleared
-    build_marks(p, r, row, c0, c1, hv, s_hkeys, s_hvals, slots, &s_full);
+    build_marks(p, r, row, c0, c1, hv, s_hkeys, s_hvals, slots, ids > (uint32_t)kHashSlots, &s_full);
   }
 
   process_unit<DT, SLOTS, VEC, MASK, WB>(p, row, chunk, r, raw, mw, s_x, s_hkeys, s_hvals, slots, &s_full);
@@ -1133,17 +1149,17 @@ __device__ __forceinline__ uint32_t record_select_row(const Params& p, const Row
   if (r.use_hist) {
     const uint32_t* win = p.history + (size_t)row * p.history_ld + r.wstart;
     for (uint32_t j = tid; j < r.wn; j += kThreads)
-      if (win[j] < p.V) hash_insert_from(hk, hv, kRecHash, win[j], 1u, 0u);
+      if (win[j] < p.V) hash_insert_from(hk, hv, kRecHash, kRecHash, win[j], 1u, 0u);
   }
   for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
     const uint32_t id = p.ban_ids[r.ban_off + k];
-    if (id < p.V) hash_insert_from(hk, hv, kRecHash, id, 0u, kBanFlag);
+    if (id < p.V) hash_insert_from(hk, hv, kRecHash, kRecHash, id, 0u, kBanFlag);
   }
   for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
     const uint32_t id = p.bias_ids[r.bias_off + k];
-    if (id < p.V) hash_insert_from(hk, hv, kRecHash, id, 0u, kBiasFlag);
+    if (id < p.V) hash_insert_from(hk, hv, kRecHash, kRecHash, id, 0u, kBiasFlag);
   }
-  if (tid == 0 && r.nl_active) hash_insert_from(hk, hv, kRecHash, r.nl_id, 0u, kNlFlag);
+  if (tid == 0 && r.nl_active) hash_insert_from(hk, hv, kRecHash, kRecHash, r.nl_id, 0u, kNlFlag);
   __syncthreads();
   const auto push = [&](uint64_t key) {
     const uint32_t q = atomicAdd(&ts.counter, 1u);

@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 
 from harness import compare, run_gpu, run_oracle
-from oxide_sampler import MirostatMode
+from oxide_sampler import MirostatMode, configs_to_array
 from oxide_sampler import workloads as wl
 
 RTOL_F32 = 1e-5
@@ -177,6 +177,49 @@ def test_penalty_ids_at_the_sizes_of_the_chunk_hash(torch_gpu, n):
         g = run_gpu(w, torch_gpu, logits_out=out, record=False, max_top_k=300)
         r = run_oracle(w, logits_out=out, record=False)
         compare(g, r, RTOL_F32, w.name)
+
+
+@pytest.mark.gpu
+def test_ids_past_the_chunk_hash_cost_no_full_probes(torch_gpu):
+    # more distinct window ids in a chunk than its hash takes: the answers are the oracle's, and the row's
+    # cost grows with the window it reads, not with the slots its failing insertions look at. (A row of
+    # 30000 ids takes 3.1 times as long as one of 1000; 13 times when each insertion probed a full table.)
+    rng = np.random.default_rng(5)
+    cfg = wl.disabled_config(repeat_penalty=1.1, repeat_last_n=0, temperature=0.8, top_k=40, top_p=0.95)
+    w = wl.Workload(name="3000 ids in a chunk", logits=(rng.standard_normal((2, 5000)) * 2.0).astype(np.float32),
+                    dtype="f32", configs=[cfg] * 2,
+                    history=np.stack([rng.permutation(5000)[:3000].astype(np.uint32) for _ in range(2)]),
+                    history_len=np.full(2, 3000, np.uint32), uniforms=wl.xorshift_uniforms(2, 5))
+    banner("windows past the chunk hash")
+    compare(run_gpu(w, torch_gpu, record=False), run_oracle(w, record=False), RTOL_F32, w.name)
+
+    from harness import gpu_sampler
+    torch, B, V = torch_gpu, 64, 128256
+    g = torch.Generator(device="cuda").manual_seed(5)
+    logits = torch.randn(B, V, generator=g, device="cuda") * 2.0
+    raw, _, _, _ = configs_to_array([cfg] * B, 10)
+    configs = torch.from_numpy(raw).cuda()
+    u = torch.full((B,), 0.5, device="cuda")
+    s = gpu_sampler(B, V, exact_limits=True)
+
+    def milliseconds(n):
+        hist = torch.stack([torch.randperm(32000, generator=g, device="cuda")[:n] if n > 1024 else
+                            torch.randperm(1024, generator=g, device="cuda")[:n] for _ in range(B)])
+        hist = hist.to(torch.int32).contiguous()
+        hlen = torch.full((B,), n, dtype=torch.int32, device="cuda")
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            s.sample(logits, configs, history=hist, history_len=hlen, history_cap=n, record=False, uniforms=u)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    few, many = milliseconds(1000), milliseconds(30000)
+    print(f"1000 ids {few:.3f} ms, 30000 ids {many:.3f} ms", flush=True)
+    assert many < 6.0 * few, (few, many)
 
 
 @pytest.mark.gpu
