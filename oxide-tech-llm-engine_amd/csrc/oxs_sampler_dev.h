@@ -452,45 +452,50 @@ __device__ uint32_t block_excl_scan(uint32_t v, uint32_t* total, uint32_t* scrat
 
 // A stream block marks the sparse-stage ids of its chunk (history window
 // with counts, bans, biases, newline) in an open-addressing LDS hash keyed by
-// chunk offset.
+// chunk offset. The table takes 256, 512 or 1024 slots by the row's ids. Most
+// chunks hold few of a row's ids, so a row of up to one and a half times as many
+// ids as slots tries the smaller table; the chunk that holds more than it takes (a window
+// skewed to one chunk: a sixteenth of the vocabulary can hold 400 of a 1024-id
+// window's ids) builds its marks again in the whole one. An overflow of the whole
+// one sends the row to the tail's exact re-scan.
 //
-// The table takes as many slots as the row has sparse-stage ids, in steps of
-// 64 (a wavefront's visit), at least kHashMin and at most kHashSlots: it then holds every id of a row of up to 960 of
-// them, however skewed to one chunk. With 256 slots a window of 1024 ids, a
-// third of them in the vocabulary's first chunk, overflowed the table there,
-// and an overflow sends the whole row to the tail's exact re-scan: 256 rows of
-// 151936 bf16 logits took 2947 us, and take 57 with the table sized by the row
-// (64 rows x 128256, 512-id windows: 20.9 -> 18.9; one row x 32000, 64 ids: 12.8 -> 12.9 or
-// 13.0 -> 13.0; 512 rows x 262144, 257-id windows: 94.0 -> 95.6 or 94.5 -> 95.1, a
-// fifth wavefront visit and the longer slot arithmetic).
-// 960 slots beside the 32 KB of staged values stay within a quarter of the
-// CU's 160 KB of LDS, so four blocks stay resident. Rows of up to 256 ids
-// visit 256 slots only; clearing all 960 is two 16-byte stores per thread
-// while the row's record is on its way.
-constexpr int kHashSlots = 960;
-constexpr int kHashMin = kThreads;  // a slot per thread
-constexpr uint32_t kHashProbes = 128;  // slots an insertion of a row with more ids than the table looks at
+// Rows of up to kHashTry ids have code of their own, with the table's size a
+// constant, that falls through: with many blocks this kernel is bound by instruction
+// issue, and about 20 instructions per wavefront are 2% of it.
+// Measured, us, one table of 256 / 256 to 960 slots by the row's ids, scaled / this:
+// 256 rows x 151936 bf16, 256 ids 36.1 / 37.0 / 36.3, 513 ids 39.3 / 39.1 / 38.8;
+// 512 x 262144, 300 ids 92.8 / 94.7 / 93.3; 64 x 128256, 512 ids 20.4 / 17.2 / 17.3;
+// 64 x 128256, 900 distinct ids in one chunk 780 / 38 / 23.
+// 1024 slots beside the 32 KB of staged values are a quarter of the CU's 160 KB of
+// LDS, so four blocks stay resident; the overflow mark is the last slot's value.
+constexpr uint32_t kHashBits = 10;
+constexpr uint32_t kHashSlots = 1u << kHashBits;  // the whole table
+constexpr uint32_t kHashIds = kHashSlots - 1u;    // ids it holds
+constexpr uint32_t kHashSmall = 256;              // the smallest table: a slot per thread
+constexpr uint32_t kHashTry = 384;                // rows of up to this many ids try the smallest table, ...
+constexpr uint32_t kHashTryMid = 768;             // ... this many the one of 512
+constexpr uint32_t kHashProbes = 128;             // slots an insertion looks at where the table may fill up
 constexpr uint32_t kEmptySlot = 0xffffffffu;
-static_assert(kHashSlots % 4 == 0 && kHashSlots / 4 <= kThreads, "cleared by one 16-byte store per thread");
-static_assert((kMaxChunk + 2 * kHashSlots) * 4 + 64 <= 160 * 1024 / 4, "four stream blocks per CU");
-// The row's sparse-stage ids, counted up to one more than the hash takes.
+constexpr uint32_t kTakenSlot = 0xfffffffeu;  // the whole table's last slot: no chunk offset
+static_assert(kHashSmall == kThreads && kHashSlots == 4 * kThreads, "slots per thread");
+static_assert(kHashTryMid <= kHashIds, "marks built again fit the whole table");
+static_assert((kMaxChunk + 2 * kHashSlots) * 4 <= 160 * 1024 / 4, "four stream blocks per CU");
+// The row's sparse-stage ids. (A sum past 2^32 only costs time: an id that finds no slot sets the mark.)
 __device__ __forceinline__ uint32_t hash_ids_of(const RowXf& r) {
-  const uint32_t most = (uint32_t)kHashSlots + 1u;
-  return min((r.use_hist ? min(r.wn, most) : 0u) + min(r.ban_cnt, most) + min(r.bias_cnt, most) +
-                 (r.nl_active ? 1u : 0u),
-             most);
+  return (r.use_hist ? r.wn : 0u) + r.ban_cnt + r.bias_cnt + (r.nl_active ? 1u : 0u);
 }
-__device__ __forceinline__ uint32_t hash_slots_of(uint32_t ids) {
-  return max((uint32_t)kHashMin, min((ids + 63u) & ~63u, (uint32_t)kHashSlots));
+// log2 of the slots for that many ids.
+__device__ __forceinline__ uint32_t hash_bits_of(uint32_t ids) {
+  return ids <= kHashTry ? 8u : ids <= kHashTryMid ? 9u : kHashBits;
 }
-__device__ __forceinline__ uint32_t hash_slot(uint32_t key, uint32_t slots) {
-  return __umul24((key * 0x9e3779b1u) >> 16, slots) >> 16;  // (slots <= 2048)
+__device__ __forceinline__ uint32_t hash_slot(uint32_t key, uint32_t bits) {
+  return (key * 0x9e3779b1u) >> (32u - bits);
 }
 
 // Continues an insertion whose home slot held another key; false when `probes` slots held others.
-__device__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t slots, uint32_t probes, uint32_t key,
-                                 uint32_t add, uint32_t orv) {
-  uint32_t h = hash_slot(key, slots);
+__device__ __forceinline__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t bits, uint32_t probes,
+                                                 uint32_t key, uint32_t add, uint32_t orv) {
+  uint32_t h = hash_slot(key, bits);
   for (uint32_t probe = 0; probe < probes; ++probe) {
     const uint32_t prev = atomicCAS(&hkeys[h], kEmptySlot, key);
     if (prev == kEmptySlot || prev == key) {
@@ -498,12 +503,97 @@ __device__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t slot
       if (orv) atomicOr(&hvals[h], orv);
       return true;
     }
-    h = h + 1u == slots ? 0u : h + 1u;
+    h = (h + 1u) & ((1u << bits) - 1u);
   }
   return false;
 }
 
 // ---------------------------------------------------------------- stream kernel
+
+// The chunk's sparse-stage ids into the LDS hash: a count per
+// history window occurrence, a flag per ban, bias and newline. The first claim
+// of every window id's home slot goes out at once, collisions after. Ends
+// with no barrier: the next block barrier completes the marks.
+// BITS: log2 of the table's slots where it is constant, else 0.
+//
+// Where the row has more ids than the table takes, insertions give up after
+// kHashProbes slots, and a long window is left once one has given up.
+// 64 rows x 128256, windows of 30000 distinct ids: 2264 us (13057 with every
+// insertion looking at a full table of 960 slots).
+template <uint32_t BITS>
+__device__ __forceinline__ void build_marks(const Params& p, const RowXf& r, uint32_t row, uint32_t c0,
+                                            uint32_t c1, const uint32_t (&hv)[kHistUnroll], uint32_t* s_hkeys,
+                                            uint32_t* s_hvals, uint32_t ids, uint32_t* s_full) {
+  const uint32_t tid = threadIdx.x;
+  const uint32_t bits = BITS ? BITS : hash_bits_of(ids);
+  const uint32_t probes = BITS || ids < 1u << bits ? 1u << bits : kHashProbes;
+  bool ok = true;
+  const auto insert = [&](uint32_t key, uint32_t add, uint32_t orv) {
+    ok &= hash_insert_from(s_hkeys, s_hvals, bits, probes, key, add, orv);
+  };
+  uint32_t prev[kHistUnroll];
+#pragma unroll
+  for (int q = 0; q < kHistUnroll; ++q) {
+    const uint32_t t = r.use_hist && tid + q * kThreads < r.wn ? hv[q] : 0xffffffffu;
+    const bool in = t >= c0 && t < c1;
+    prev[q] = in ? atomicCAS(&s_hkeys[hash_slot(t - c0, bits)], kEmptySlot, t - c0) : 0u;
+  }
+#pragma unroll
+  for (int q = 0; q < kHistUnroll; ++q) {
+    const uint32_t t = r.use_hist && tid + q * kThreads < r.wn ? hv[q] : 0xffffffffu;
+    if (!(t >= c0 && t < c1)) continue;
+    if (prev[q] == kEmptySlot || prev[q] == t - c0) atomicAdd(&s_hvals[hash_slot(t - c0, bits)], 1u);
+    else insert(t - c0, 1u, 0u);
+  }
+  if (!BITS && r.use_hist) {  // long windows
+    const uint32_t* hrow = p.history + (size_t)row * p.history_ld + r.wstart;
+    for (uint32_t j = tid + kHistUnroll * kThreads; j < r.wn; j += kThreads) {
+      // (an atomic load: a volatile one would go through a flat address and wait for the logits)
+      if (!ok) *s_full = 1;
+      if (__hip_atomic_load(s_full, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
+      const uint32_t t = hrow[j];
+      if (t >= c0 && t < c1) insert(t - c0, 1u, 0u);
+    }
+  }
+  for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
+    const uint32_t id = p.ban_ids[r.ban_off + k];
+    if (id >= c0 && id < c1) insert(id - c0, 0u, kBanFlag);
+  }
+  for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
+    const uint32_t id = p.bias_ids[r.bias_off + k];
+    if (id >= c0 && id < c1) insert(id - c0, 0u, kBiasFlag);
+  }
+  if (tid == 0 && r.nl_active && r.nl_id >= c0 && r.nl_id < c1) insert(r.nl_id - c0, 0u, kNlFlag);
+  if (!ok) *s_full = 1;
+}
+
+// Clears the table from slot `from` on; its last slot is taken.
+__device__ __forceinline__ void clear_marks(uint32_t* s_hkeys, uint32_t* s_hvals, uint32_t from) {
+  const uint32_t h = 4u * threadIdx.x;
+  if (h < from) return;
+  *(uint4*)&s_hkeys[h] = make_uint4(kEmptySlot, kEmptySlot, kEmptySlot, h + 4u == kHashSlots ? kTakenSlot : kEmptySlot);
+  *(uint4*)&s_hvals[h] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// The marks again in the whole table, for a chunk with more distinct ids than the smaller one
+// takes (of a row of at most kHashTryMid: every id finds a slot).
+__device__ __forceinline__ void rebuild_marks(const Params& p, const RowXf& r, uint32_t row, uint32_t c0,
+                                              uint32_t c1, uint32_t* s_hkeys, uint32_t* s_hvals) {
+  const uint32_t tid = threadIdx.x;
+  clear_marks(s_hkeys, s_hvals, 0u);
+  __syncthreads();
+  const uint32_t wn = r.use_hist ? r.wn : 0u, n1 = wn + r.ban_cnt, n2 = n1 + r.bias_cnt;
+  const uint32_t n = n2 + (r.nl_active ? 1u : 0u);
+#pragma unroll 1
+  for (uint32_t j = tid; j < n; j += kThreads) {
+    uint32_t id = r.nl_id, flag = kNlFlag;
+    if (j < wn) id = p.history[(size_t)row * p.history_ld + r.wstart + j], flag = 0u;
+    else if (j < n1) id = p.ban_ids[r.ban_off + (j - wn)], flag = kBanFlag;
+    else if (j < n2) id = p.bias_ids[r.bias_off + (j - n1)], flag = kBiasFlag;
+    if (id >= c0 && id < c1) hash_insert_from(s_hkeys, s_hvals, kHashBits, kHashSlots, id - c0, flag ? 0u : 1u, flag);
+  }
+  __syncthreads();
+}
 
 constexpr uint32_t kMinValidOrd = 0x00800000u;  // f2ord(-FLT_MAX): every candidate key is >= this
 
@@ -520,8 +610,8 @@ constexpr uint32_t kMinValidOrd = 0x00800000u;  // f2ord(-FLT_MAX): every candid
 template <int DT, int SLOTS, bool VEC, bool MASK, bool WB>
 __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint32_t chunk, const RowXf& r,
                                              const uint32_t (&raw)[SLOTS][kind_f32(DT) ? 4 : 8],
-                                             const uint32_t (&mw)[SLOTS], float* s_x, uint32_t* s_hkeys,
-                                             uint32_t* s_hvals, uint32_t slots, uint32_t* s_full) {
+                                             const uint32_t (&mw)[SLOTS], float* s_x,
+                                             uint32_t* s_hkeys, uint32_t* s_hvals, uint32_t ids, uint32_t* s_full) {
   constexpr int EPL = kind_f32(DT) ? 4 : 8;
   constexpr int TILE = kThreads * EPL;
   constexpr int NE = SLOTS * EPL;
@@ -563,10 +653,29 @@ __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint
   // ---- sparse-stage ids at their exact values (sampler.rs:184-245)
   if (r.any_special) {
     __syncthreads();  // values staged, marks complete
-    for (uint32_t h = tid; h < slots; h += kThreads) {
-      const uint32_t off = s_hkeys[h];
-      if (off != kEmptySlot) s_x[off] = apply_special(p.bias_ids, p.bias_values, r, s_x[off], s_hvals[h], c0 + off);
+    // the slots of a thread: one, or two or four in a row
+    uint32_t h = tid, turns = 1;
+    uint4 k;
+    if (__builtin_expect(ids > kHashSmall, 0)) {
+      uint32_t bits = hash_bits_of(ids);
+      if (ids <= kHashTryMid && *s_full != 0u) {
+        __syncthreads();  // (every wavefront has read the mark)
+        rebuild_marks(p, r, row, c0, c1, s_hkeys, s_hvals);
+        bits = kHashBits;
+      }
+      turns = 1u << (bits - 8u);
+      h = tid * turns;
+      if (bits > 8u) k = *(const uint4*)&s_hkeys[bits == 9u ? h & ~3u : h];
+      if (bits == 9u && (tid & 1u)) k.x = k.z, k.y = k.w;
     }
+    if (turns == 1u) k.x = s_hkeys[tid];
+#pragma unroll 1
+    do {  // (block-uniform turns)
+      const uint32_t off = k.x;
+      if (off < CH) s_x[off] = apply_special(p.bias_ids, p.bias_values, r, s_x[off], s_hvals[h], c0 + off);
+      if (--turns == 0u) break;
+      ++h, k.x = k.y, k.y = k.z, k.z = k.w;
+    } while (true);
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s)
@@ -661,60 +770,6 @@ __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint
   }
 }
 
-// The chunk's sparse-stage ids into the LDS hash: a count per
-// history window occurrence, a flag per ban, bias and newline. The first claim
-// of every window id's home slot goes out at once, collisions after. Ends
-// with no barrier: the next block barrier completes the marks.
-//
-// A row with more ids than the table takes may fill it. Its insertions give up
-// after kHashProbes slots (the table is then full, or so nearly that the row
-// goes to the exact re-scan anyway), and nothing more is inserted once one has
-// given up. 64 rows x 128256: windows of 30000 distinct ids 2257 us (13064 with
-// every failing insertion looking at all 960 slots), of 1000 in 1024 733 (991).
-__device__ __forceinline__ void build_marks(const Params& p, const RowXf& r, uint32_t row, uint32_t c0,
-                                            uint32_t c1, const uint32_t (&hv)[kHistUnroll],
-                                            uint32_t* s_hkeys, uint32_t* s_hvals, uint32_t slots, bool many, uint32_t* s_full) {
-  const uint32_t tid = threadIdx.x;
-  const uint32_t probes = many ? kHashProbes : slots;
-  volatile uint32_t* full = s_full;
-  const auto insert = [&](uint32_t key, uint32_t add, uint32_t orv) {
-    if (many && *full) return;
-    if (!hash_insert_from(s_hkeys, s_hvals, slots, probes, key, add, orv)) *full = 1;
-  };
-  uint32_t prev[kHistUnroll];
-#pragma unroll
-  for (int q = 0; q < kHistUnroll; ++q) {
-    const uint32_t t = r.use_hist && tid + q * kThreads < r.wn ? hv[q] : 0xffffffffu;
-    const bool in = t >= c0 && t < c1;
-    prev[q] = in ? atomicCAS(&s_hkeys[hash_slot(t - c0, slots)], kEmptySlot, t - c0) : 0u;
-  }
-#pragma unroll
-  for (int q = 0; q < kHistUnroll; ++q) {
-    const uint32_t t = r.use_hist && tid + q * kThreads < r.wn ? hv[q] : 0xffffffffu;
-    if (!(t >= c0 && t < c1)) continue;
-    if (prev[q] == kEmptySlot || prev[q] == t - c0) atomicAdd(&s_hvals[hash_slot(t - c0, slots)], 1u);
-    else insert(t - c0, 1u, 0u);
-  }
-  if (r.use_hist) {
-    const uint32_t* hrow = p.history + (size_t)row * p.history_ld + r.wstart;
-    for (uint32_t j = tid + kHistUnroll * kThreads; j < r.wn; j += kThreads) {  // long windows
-      if (many && *full) break;
-      const uint32_t t = hrow[j];
-      if (t >= c0 && t < c1) insert(t - c0, 1u, 0u);
-    }
-  }
-  for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
-    const uint32_t id = p.ban_ids[r.ban_off + k];
-    if (id >= c0 && id < c1) insert(id - c0, 0u, kBanFlag);
-  }
-  for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
-    const uint32_t id = p.bias_ids[r.bias_off + k];
-    if (id >= c0 && id < c1) insert(id - c0, 0u, kBiasFlag);
-  }
-  if (tid == 0 && r.nl_active && r.nl_id >= c0 && r.nl_id < c1)
-    insert(r.nl_id - c0, 0u, kNlFlag);
-}
-
 // One (row, chunk) per block. The first half of the chunk's logits is issued
 // at once (its addresses need nothing from memory); the row's record comes
 // through the scalar cache meanwhile; then the history window ids and the
@@ -743,7 +798,7 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
   __shared__ __align__(16) float s_x[NE * kThreads];  // each thread's masked raw logits (private slots)
   __shared__ __align__(16) uint32_t s_hkeys[kHashSlots];
   __shared__ __align__(16) uint32_t s_hvals[kHashSlots];
-  __shared__ uint32_t s_full;
+  uint32_t* s_full = s_hvals + kHashIds;
 
   const uint32_t tid = threadIdx.x;
   // the block's (row, chunk). With rpx > 0 the hardware's round-robin
@@ -799,11 +854,9 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
       mw[s] = p.mask[(size_t)row * p.mask_ld + ((b2 < c1 ? b2 : p.V - 1) >> 5)];
     }
   }
-  if (tid < (uint32_t)kHashSlots / 4u) {
-    *(uint4*)&s_hkeys[4 * tid] = make_uint4(kEmptySlot, kEmptySlot, kEmptySlot, kEmptySlot);
-    *(uint4*)&s_hvals[4 * tid] = make_uint4(0u, 0u, 0u, 0u);
-  }
-  if (tid == 0) s_full = 0;
+  s_hkeys[tid] = kEmptySlot;
+  s_hvals[tid] = 0u;
+  if (tid == 0) *s_full = 0u;
   __builtin_amdgcn_sched_barrier(0);
   oxs_sampling_config cfg;
   {
@@ -815,7 +868,6 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
   const uint32_t hlen = (uint32_t)__builtin_amdgcn_readlane((int)rec, 26);
   if ((kflags & kKDecode) && cfg.temperature <= 1e-6f) raw_argmax_config(cfg);  // continuous_batching.rs:961
   const RowXf r = make_row_xf(cfg, hlen, V, history_ld, kflags);
-  const uint32_t ids = hash_ids_of(r), slots = hash_slots_of(ids);
   // history window ids, read without a branch (an in-bounds dummy address
   // where the row has none)
   uint32_t hv[kHistUnroll];
@@ -838,12 +890,20 @@ __global__ __launch_bounds__(kThreads) void stream_kernel(const void* __restrict
 #pragma unroll
       for (int e = 0; e < EPL; ++e) raw[s][e] = __float_as_uint(softcap_of(__uint_as_float(raw[s][e]), p.softcap));
   }
+  uint32_t ids = 0;
   if (r.any_special) {
-    __syncthreads();  // tables cleared
-    build_marks(p, r, row, c0, c1, hv, s_hkeys, s_hvals, slots, ids > (uint32_t)kHashSlots, &s_full);
+    ids = hash_ids_of(r);
+    if (__builtin_expect(ids <= kHashTry, 1)) {
+      __syncthreads();  // table cleared
+      build_marks<8>(p, r, row, c0, c1, hv, s_hkeys, s_hvals, ids, s_full);
+    } else {
+      clear_marks(s_hkeys, s_hvals, kHashSmall);
+      __syncthreads();
+      build_marks<0>(p, r, row, c0, c1, hv, s_hkeys, s_hvals, ids, s_full);
+    }
   }
 
-  process_unit<DT, SLOTS, VEC, MASK, WB>(p, row, chunk, r, raw, mw, s_x, s_hkeys, s_hvals, slots, &s_full);
+  process_unit<DT, SLOTS, VEC, MASK, WB>(p, row, chunk, r, raw, mw, s_x, s_hkeys, s_hvals, ids, s_full);
 }
 
 // ---------------------------------------------------------------- tail helpers
@@ -1103,7 +1163,7 @@ __device__ __forceinline__ uint32_t exact_select_row(const Params& p, const RowX
 // a write-back (the radix select repairs it), more ids than the hash takes,
 // thresholds that bound too few keys (few wavefronts and a large M), more keys
 // than fit. area: kTailArea words; rec: 3 * kThreads words.
-constexpr int kRecHash = 2048;  // row-wide slots of sparse-stage ids (a key and an entry each)
+constexpr int kRecBits = 11, kRecHash = 1 << kRecBits;  // row-wide slots of sparse-stage ids (a key and an entry each)
 constexpr int kRecIds = 1536;   // ids at most
 constexpr int kRecCands = 2048;
 static_assert(kRecHash + kRecCands <= kTailArea && kMaxM <= kRecCands, "record selection fits the key area");
@@ -1149,24 +1209,24 @@ __device__ __forceinline__ uint32_t record_select_row(const Params& p, const Row
   if (r.use_hist) {
     const uint32_t* win = p.history + (size_t)row * p.history_ld + r.wstart;
     for (uint32_t j = tid; j < r.wn; j += kThreads)
-      if (win[j] < p.V) hash_insert_from(hk, hv, kRecHash, kRecHash, win[j], 1u, 0u);
+      if (win[j] < p.V) hash_insert_from(hk, hv, kRecBits, kRecHash, win[j], 1u, 0u);
   }
   for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
     const uint32_t id = p.ban_ids[r.ban_off + k];
-    if (id < p.V) hash_insert_from(hk, hv, kRecHash, kRecHash, id, 0u, kBanFlag);
+    if (id < p.V) hash_insert_from(hk, hv, kRecBits, kRecHash, id, 0u, kBanFlag);
   }
   for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
     const uint32_t id = p.bias_ids[r.bias_off + k];
-    if (id < p.V) hash_insert_from(hk, hv, kRecHash, kRecHash, id, 0u, kBiasFlag);
+    if (id < p.V) hash_insert_from(hk, hv, kRecBits, kRecHash, id, 0u, kBiasFlag);
   }
-  if (tid == 0 && r.nl_active) hash_insert_from(hk, hv, kRecHash, kRecHash, r.nl_id, 0u, kNlFlag);
+  if (tid == 0 && r.nl_active) hash_insert_from(hk, hv, kRecBits, kRecHash, r.nl_id, 0u, kNlFlag);
   __syncthreads();
   const auto push = [&](uint64_t key) {
     const uint32_t q = atomicAdd(&ts.counter, 1u);
     if (q < (uint32_t)kRecCands) cand[q] = key;
   };
   const auto special = [&](uint32_t id) {
-    for (uint32_t h = hash_slot(id, kRecHash); hk[h] != kEmptySlot; h = (h + 1u) & (kRecHash - 1u))
+    for (uint32_t h = hash_slot(id, kRecBits); hk[h] != kEmptySlot; h = (h + 1u) & (kRecHash - 1u))
       if (hk[h] == id) return true;
     return false;
   };

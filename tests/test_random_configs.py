@@ -180,10 +180,46 @@ def test_penalty_ids_at_the_sizes_of_the_chunk_hash(torch_gpu, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [256, 257, 384, 385, 512, 513, 768, 769, 1000, 1023, 1024, 3000])
+def test_skewed_windows_keep_the_candidate_path(torch_gpu, n):
+    # n distinct window ids in the first of 16 stream chunks, with bans, biases and repeats among them:
+    # up to 1023 the chunk's marks fit its hash (built again from 257 on where a smaller one was tried)
+    # and the row keeps the candidate path; more overflow it and the row is re-scanned, which also
+    # repairs logits_out
+    rng = np.random.default_rng(n)
+    B, V = 4, 128256
+    logits = (rng.standard_normal((B, V)) * 2.0).astype(np.float32)
+    ids = np.stack([rng.permutation(8192)[:n].astype(np.uint32) for _ in range(B)])
+    history = np.concatenate([ids, ids[:, : n // 8]], axis=1) if n in (257, 769) else ids
+    configs = []
+    for i in range(B):
+        c = wl.disabled_config(frequency_penalty=0.3, presence_penalty=0.2, repeat_penalty=1.2, repeat_last_n=0,
+                               temperature=0.7, top_k=50, top_p=0.9)
+        if i % 2 and n < 1023:  # of the window's own ids, so that the chunk's distinct ids stay n
+            c.banned_tokens = {int(t) for t in ids[i, :3]}
+            c.logit_biases = {int(t): 1.5 for t in ids[i, 2:5]}
+        configs.append(c)
+    w = wl.Workload(name=f"{n} ids in one chunk", logits=logits, dtype="f32", configs=configs, history=history,
+                    history_len=np.full(B, history.shape[1], np.uint32), uniforms=wl.xorshift_uniforms(B, n))
+    banner(w.name)
+    from harness import gpu_sampler
+    for out in (True, False):
+        s = gpu_sampler(B, V, exact_limits=True)
+        s.count_paths(True)
+        try:
+            g = run_gpu(w, torch_gpu, logits_out=out, record=False, exact_limits=True)
+            counts = s.path_counts()
+        finally:
+            s.count_paths(False)
+        compare(g, run_oracle(w, logits_out=out, record=False), RTOL_F32, w.name)
+        assert counts["exact"] == (0 if n <= 1023 else B), counts
+
+
+@pytest.mark.gpu
 def test_ids_past_the_chunk_hash_cost_no_full_probes(torch_gpu):
     # more distinct window ids in a chunk than its hash takes: the answers are the oracle's, and the row's
     # cost grows with the window it reads, not with the slots its failing insertions look at. (A row of
-    # 30000 ids takes 3.1 times as long as one of 1000; 13 times when each insertion probed a full table.)
+    # 30000 ids takes 3.1 times as long as one of 1100; 13 times when each insertion probed a full table.)
     rng = np.random.default_rng(5)
     cfg = wl.disabled_config(repeat_penalty=1.1, repeat_last_n=0, temperature=0.8, top_k=40, top_p=0.95)
     w = wl.Workload(name="3000 ids in a chunk", logits=(rng.standard_normal((2, 5000)) * 2.0).astype(np.float32),
@@ -202,9 +238,8 @@ def test_ids_past_the_chunk_hash_cost_no_full_probes(torch_gpu):
     u = torch.full((B,), 0.5, device="cuda")
     s = gpu_sampler(B, V, exact_limits=True)
 
-    def milliseconds(n):
-        hist = torch.stack([torch.randperm(32000, generator=g, device="cuda")[:n] if n > 1024 else
-                            torch.randperm(1024, generator=g, device="cuda")[:n] for _ in range(B)])
+    def milliseconds(n, span):
+        hist = torch.stack([torch.randperm(span, generator=g, device="cuda")[:n] for _ in range(B)])
         hist = hist.to(torch.int32).contiguous()
         hlen = torch.full((B,), n, dtype=torch.int32, device="cuda")
         best = float("inf")
@@ -217,8 +252,8 @@ def test_ids_past_the_chunk_hash_cost_no_full_probes(torch_gpu):
             best = min(best, a.elapsed_time(b))
         return best
 
-    few, many = milliseconds(1000), milliseconds(30000)
-    print(f"1000 ids {few:.3f} ms, 30000 ids {many:.3f} ms", flush=True)
+    few, many = milliseconds(1100, 2048), milliseconds(30000, 32000)
+    print(f"1100 ids {few:.3f} ms, 30000 ids {many:.3f} ms", flush=True)
     assert many < 6.0 * few, (few, many)
 
 
