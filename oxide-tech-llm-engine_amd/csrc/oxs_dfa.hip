@@ -21,6 +21,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/oxide_sampler.h"
 
 namespace oxs_grammar {
@@ -30,6 +32,7 @@ constexpr int kTok = 2;               // tokens per thread
 constexpr int kWords = kTok * kThreads / 32;  // mask words per row and block
 constexpr int kRows = 128;            // rows per block with a walk from every state
 constexpr uint32_t kList = 64;        // start states walked together
+constexpr int kIlp = 4;               // of them, by one thread at the same time
 constexpr uint32_t kPermStates = 8;   // tables whose transition functions fit a byte permute
 constexpr uint32_t kLdsStates = 128;  // tables of up to 128 states are kept in LDS, a byte per entry
 constexpr uint32_t kErr = OXS_DFA_ERROR_STATE;
@@ -90,10 +93,11 @@ __device__ __forceinline__ void load_piece(const Params& p, uint32_t at, uint32_
 // are the table's own (num_states <= 64) and blockIdx.y picks kRows rows;
 // otherwise they are the states of the 64 rows that blockIdx.y picks.
 //
-// Measured, 128 rows x 128256 tokens, us per launch (in brackets: a walk of
-// every state per 32 rows or of every row per 16, byte loads and a ballot per
-// row): 8 states 7.3 (25.8), 16 states 16.9 (31.9), 64 states 32.8 (93.8), 69
-// states 41.6 (62.7), 154 states 30.5 (58.6); 8 rows, 64 states 9.7 (86.2).
+// Measured, us per launch, in brackets with one walk after the other per thread:
+// 128 rows x 128256 tokens, a fixed-prefix grammar (few start states accept a first
+// byte) of 8 states 7.7 (walks nothing), 16 states 13.0 (17.6), 64 states 25.7 (32.9), 129
+// states 22.9 (28.3); tables without error entries of 16 states 24.9 (57.5), 300
+// states 208 (376). One row, 64 states 8.4 (8.3).
 template <Walk WALK>
 __global__ __launch_bounds__(kThreads) void dfa_mask_kernel(const Params p, const uint32_t by_state) {
   extern __shared__ __align__(16) uint8_t s_table[];  // kLds: [num_states][256] next states
@@ -197,33 +201,51 @@ __global__ __launch_bounds__(kThreads) void dfa_mask_kernel(const Params p, cons
       if (len[k] == 1u) {
         alive = todo;
       } else {
-        while (todo) {  // the start states that accept the first byte
-          const uint32_t i = (uint32_t)__builtin_ctzll(todo);
-          todo &= todo - 1u;
-          uint32_t c = s_start[i];
-          bool ok = true;
-          for (uint32_t j0 = 0; j0 < len[k] && ok; j0 += 16u) {
+        // the start states that accept the first byte. A walk is a chain of
+        // dependent reads, so kIlp of them are kept in flight while any token of the
+        // wavefront has more than one left.
+        constexpr uint32_t dead = WALK == kLds ? kDead : kErr;
+        const auto walk = [&](auto ilp) {
+          constexpr int ILP = decltype(ilp)::value;
+          uint32_t c[ILP];
+          uint64_t bit[ILP];
+#pragma unroll
+          for (int e = 0; e < ILP; ++e) {
+            bit[e] = todo & (0ull - todo);
+            c[e] = todo ? s_start[__builtin_ctzll(todo)] : dead;
+            todo &= todo - 1ull;
+          }
+          for (uint32_t j0 = 0; j0 < len[k]; j0 += 16u) {
             uint32_t w[4] = {piece[k][0], piece[k][1], piece[k][2], piece[k][3]};
             if (j0) load_piece(p, b0[k] + j0, w);
             const uint32_t n = min(len[k] - j0, 16u);
+            bool any = true;
 #pragma unroll
             for (uint32_t j = 0; j < 16; ++j) {
-              if (j < n && ok) {  // (DfaSchemaGrammar::transition, dfa.rs:110-126)
+              if (j < n && any) {  // (DfaSchemaGrammar::transition, dfa.rs:110-126)
                 const uint32_t b = (w[j / 4] >> (8u * (j % 4u))) & 0xffu;
-                if (c >= ns) {
-                  ok = false;
-                } else if constexpr (WALK == kLds) {
-                  c = s_table[c * 256u + b];
-                  ok = c != kDead;
-                } else {
-                  c = p.trans[(size_t)c * 256u + b];
-                  ok = c != kErr;
+                uint32_t nx[ILP];
+#pragma unroll
+                for (int e = 0; e < ILP; ++e) {
+                  const uint32_t at = c[e] < ns ? c[e] : 0u;
+                  nx[e] = WALK == kLds ? s_table[at * 256u + b] : p.trans[(size_t)at * 256u + b];
                 }
+                uint32_t all = dead;
+#pragma unroll
+                for (int e = 0; e < ILP; ++e) {
+                  c[e] = c[e] < ns ? nx[e] : dead;  // (a walk outside the table fails at its next byte)
+                  all &= c[e];
+                }
+                any = all != dead;
               }
             }
+            if (!any) break;
           }
-          if (ok) alive |= 1ull << i;
-        }
+#pragma unroll
+          for (int e = 0; e < ILP; ++e) alive |= c[e] != dead ? bit[e] : 0ull;
+        };
+        while (__any((todo & (todo - 1ull)) != 0ull)) walk(std::integral_constant<int, kIlp>{});
+        if (todo) walk(std::integral_constant<int, 1>{});
       }
     }
     if (!in[k]) alive = 0;

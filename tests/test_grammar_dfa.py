@@ -194,6 +194,46 @@ def test_gpu_dfa_mask_walk_forms(torch_gpu, n, V, B, density):
 
 
 @pytest.mark.gpu
+def test_gpu_dfa_mask_dense_table_cost(torch_gpu):
+    # a table without error entries: a thread walks its token from each of 64 start states. Walked four at
+    # a time, 128 rows take 15 times as long as one row; one after the other they took 38 times as long.
+    import ctypes
+    from oxide_sampler._abi import OxsDfa, OxsTokenBytes, check, load_library
+    torch, lib, n, V = torch_gpu, load_library(), 300, 32000
+    rng = np.random.default_rng(9)
+    table = rng.integers(0, n, n * 256).astype(np.uint32)
+    lens = np.clip(rng.geometric(0.2, V), 1, 16)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    by = rng.integers(0, 256, int(off[-1])).astype(np.uint8)
+    t_table, t_off = (torch.from_numpy(a.view(np.int32)).cuda() for a in (table, off))
+    t_by = torch.from_numpy(by).cuda()
+    dfa, tb = OxsDfa(n, t_table.data_ptr()), OxsTokenBytes(V, int(off[-1]), t_off.data_ptr(), t_by.data_ptr())
+
+    def microseconds(B):
+        states = rng.integers(0, n, B).astype(np.uint32)
+        t_st = torch.from_numpy(states.view(np.int32)).cuda()
+        mask = torch.empty(B, V // 32, dtype=torch.int32, device="cuda")
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(50):
+                check(lib.oxs_dfa_mask(ctypes.byref(dfa), ctypes.byref(tb), ctypes.c_void_p(t_st.data_ptr()), B,
+                                       ctypes.c_void_p(mask.data_ptr()), V // 32, None), "oxs_dfa_mask")
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1000 / 50)
+        rows = rng.integers(0, B, min(B, 3))
+        want = oracle.dfa_mask_host(table, n, off, by, states[rows])
+        np.testing.assert_array_equal(mask.cpu().numpy().view(np.uint32)[rows], want)
+        return best
+
+    one, many = microseconds(1), microseconds(128)
+    print(f"\n[case] dense table: one row {one:.1f} us, 128 rows {many:.1f} us", flush=True)
+    assert many < 25.0 * one, (one, many)
+
+
+@pytest.mark.gpu
 def test_gpu_dfa_mask_empty_table(torch_gpu):
     # no states: every state is outside the table, so only tokens with no bytes are allowed
     vocab = [b"", b"a", b"", b"{}", b"x" * 40]
