@@ -344,7 +344,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mmvq_q8_0_kernel(float* __restr
 
 // The same product for batches of one or two columns, where a 32-column MFMA
 // tile would be almost idle (128256 x 4096: 96.0 and 93.7 us against 97.4 for
-// the MFMA kernel; at four columns it took 103.9). Each workgroup first stages the whole of x
+// the MFMA kernel), and for three or four where that kernel's tokens per workgroup
+// leave CUs idle (below). Each workgroup first stages the whole of x
 // (NC columns x every k block) in LDS, then each wavefront walks its 32
 // tokens with no further barrier: lane (j, g) takes 16 quant bytes of token j
 // per block (the packed layout's MFMA order), four dot4 products per column,
@@ -451,16 +452,31 @@ extern "C" int oxs_mmvq_q8_0(float* y, const void* w_packed, const void* x_q8_1,
   const uint32_t vec_out = (m % 4u == 0u && ((uintptr_t)y & 15u) == 0u) ? 1u : 0u;
   const uint32_t groups = (m + 31u) / 32u;
   const uint32_t gx = (groups + oxs_lm::kGroupsPerBlock - 1) / oxs_lm::kGroupsPerBlock;
-  if (batch <= 2u && (size_t)batch * (k / 32u) * 36u <= 65536u) {  // the whole of x fits in LDS
-    const uint32_t nb = k / 32u;
-    const size_t lds = (size_t)batch * nb * 36u;
-    const dim3 g1(gx);
-    if (batch == 1u)
-      hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_small_kernel<1>, g1, dim3(oxs_lm::kThreads), lds, (hipStream_t)stream, y,
+  const uint32_t nb = k / 32u;
+  const uint32_t blocks256 = (groups + 7u) / 8u;  // workgroups of 256 tokens: one per CU at a time
+  // Three or four columns take the small kernel where the MFMA kernel's second round of
+  // workgroups is little used or its start is much of a short row, us for 3 columns
+  // (MFMA / small): k = 128, m = 32000 5.0 / 3.8; above 256 workgroups k = 896, m =
+  // 128256 25.4 / 21.7, 80000 21.1 / 16.4, k = 1536 35.7 / 34.4, 29.4 / 25.1, but k = 2048,
+  // m = 128256 45.4 / 47.5; with less than half of the last round in use k = 2048, m =
+  // 134000 59.0 / 52.4, 80000 37.1 / 32.0, k = 3072 51.9 / 46.4, and past 512
+  // workgroups k = 4096, m = 134000 125 / 113; but k = 4096, m = 80000 76 / 85, and
+  // past 512 full ones k = 1152, m = 262144 61 / 63.
+  // Up to 256 workgroups MFMA wins from k = 512 on (50257 x 896 12.4 / 13.7).
+  const bool half_round = blocks256 % 256u != 0u && blocks256 % 256u < 128u;
+  const bool small4 =
+      k <= 256u || (blocks256 > 256u && (k <= 1024u || (k <= 1536u && blocks256 <= 512u) ||
+                                         (half_round && (k <= 3072u || blocks256 > 512u))));
+  const uint32_t nc = batch <= 2u ? batch : 4u;  // columns that the small kernel stages
+  if ((batch <= 2u || (batch <= 4u && small4)) && (size_t)nc * nb * 36u <= 65536u) {  // the whole of x fits in LDS
+    const size_t lds = (size_t)nc * nb * 36u;
+    const auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(gx), dim3(oxs_lm::kThreads), lds, (hipStream_t)stream, y,
                          (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb, batch);
-    else
-      hipLaunchKernelGGL(oxs_lm::mmvq_q8_0_small_kernel<2>, g1, dim3(oxs_lm::kThreads), lds, (hipStream_t)stream, y,
-                         (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb, batch);
+    };
+    if (nc == 1u) go(oxs_lm::mmvq_q8_0_small_kernel<1>);
+    else if (nc == 2u) go(oxs_lm::mmvq_q8_0_small_kernel<2>);
+    else go(oxs_lm::mmvq_q8_0_small_kernel<4>);
     return launch_status();
   }
   // Columns and tokens per workgroup. 64 columns read the weights half as often
@@ -469,15 +485,17 @@ extern "C" int oxs_mmvq_q8_0(float* y, const void* w_packed, const void* x_q8_1,
   // 197 of them. Measured, us: 64 columns / 32 columns for a batch of 64 at
   // k = 4096, 125 workgroups (m = 32000) 45.0 / 39.5, 197 (m = 50257) 61.7 / 69.4;
   // 256 / 128 tokens at a batch of 5, 125 workgroups 30.3 / 25.6, 197 42.2 / 45.6.
-  // (64 columns also need their offsets into x within 32 bits.)
+  // Rows of up to 512 weights take 128 tokens again above one round of the CUs, where
+  // a workgroup's start is much of its time: m = 128256, k = 512, batch 32 22.5 / 20.7, m = 200000
+  // 37.1 / 31.7. (64 columns also need their offsets into x within 32 bits.)
   constexpr uint64_t kEnough = 160;
-  const uint32_t nb = k / 32u;
   const auto blocks = [&](uint32_t cols, uint32_t waves) {
     return (uint64_t)((groups + waves - 1u) / waves) * ((batch + cols - 1u) / cols);
   };
   const bool wide = batch > 32u && blocks(64u, 8u) >= kEnough && (uint64_t)64u * nb * oxs_lm::kQ81Bytes <= 0xffffffffull;
   const uint32_t cols = wide ? 64u : 32u;
-  const uint32_t waves = wide || blocks(32u, 8u) >= kEnough ? 8u : 4u;
+  const uint64_t b32 = blocks(32u, 8u);
+  const uint32_t waves = wide || (b32 >= kEnough && !(k <= 512u && b32 > 256u)) ? 8u : 4u;
   const uint64_t grid = blocks(cols, waves);
   if (grid > 0x7fffffffull) return OXS_ERR_INVALID_ARGUMENT;
   auto go = [&](auto kernel) {

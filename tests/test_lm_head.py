@@ -228,6 +228,46 @@ def test_gpu_mmvq_matches_oracle(torch_gpu, m, k, batch):
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+def check_rows(torch_gpu, m, k, batch, rows):
+    """A projection against the oracle at `rows` of the head's tokens, bit for bit."""
+    from oxide_sampler import LmHeadQ8_0, quantize_q8_1
+    rng = np.random.default_rng(m + 3 * k + 7 * batch)
+    w = rng.integers(0, 256, (m, k // 32, 34), dtype=np.uint8)
+    w[:, :, :2] = rng.uniform(2e-4, 6e-4, (m, k // 32, 1)).astype(np.float16).view(np.uint8)
+    x = (rng.standard_normal((batch, k)) * 1.5).astype(np.float32)
+    print(f"\n[case] mmvq_q8_0 rows m={m} k={k} batch={batch}", flush=True)
+    got = LmHeadQ8_0(w.reshape(-1), m, k).project(quantize_q8_1(_to_dev(torch_gpu, x))).cpu().numpy()
+    some = np.ascontiguousarray(w[rows])
+    want = oracle.mmvq_q8_0_host(some.reshape(-1), oracle.quantize_q8_1_host(x).reshape(-1), len(rows), k, batch)
+    np.testing.assert_array_equal(got[:, rows].view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,batch", [
+    (33, 256, 3), (33, 384, 3), (65537, 128, 4), (65536, 512, 4), (65537, 512, 3), (65537, 1536, 4),
+    (65537, 3072, 3), (98304, 1664, 4), (131073, 3200, 3), (65537, 512, 5), (65537, 640, 33)])
+def test_gpu_mmvq_lines_of_the_dispatch(torch_gpu, m, k, batch):
+    # both sides of each line between the dot4 kernel (4 staged columns) and the matrix kernel: k = 256 and
+    # 384; 256 and 257 workgroups of 256 tokens; k = 1536 and above with more and less than half of the last
+    # round; and the matrix kernel's 128 tokens per workgroup at k = 512
+    rng = np.random.default_rng(m)
+    rows = np.unique(np.concatenate([np.arange(min(m, 40)), np.arange(m - 33, m),
+                                     rng.integers(0, m, 60)]))
+    check_rows(torch_gpu, m, k, batch, rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,batch", [
+    (40961, 640, 5), (40961, 1024, 32), (41000, 896, 17), (40961, 1152, 6), (40990, 768, 31),
+    (20481, 640, 64), (20500, 1408, 63)])
+def test_gpu_mmvq_32_columns_256_tokens(torch_gpu, m, k, batch):
+    # the form of 32 columns x 256 tokens per workgroup in its four-deep loop: 5 to 11 groups of four k blocks
+    # (every remainder of 4), one column block and two
+    rng = np.random.default_rng(m)
+    rows = np.unique(np.concatenate([np.arange(40), np.arange(m - 33, m), rng.integers(0, m, 200)]))
+    check_rows(torch_gpu, m, k, batch, rows)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,k,batch", [
     (1, 128, 3), (255, 128, 32), (256, 128, 33), (257, 256, 64), (513, 384, 34), (31, 512, 64),
