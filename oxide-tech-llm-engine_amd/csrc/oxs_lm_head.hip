@@ -497,7 +497,8 @@ extern "C" int oxs_mmvq_q8_0(float* y, const void* w_packed, const void* x_q8_1,
   const uint64_t b32 = blocks(32u, 8u);
   const uint32_t waves = wide || (b32 >= kEnough && !(k <= 512u && b32 > 256u)) ? 8u : 4u;
   const uint64_t grid = blocks(cols, waves);
-  if (grid > 0x7fffffffull) return OXS_ERR_INVALID_ARGUMENT;
+  // (the bound is on 128 tokens x 32 columns per workgroup whatever the launch takes)
+  if ((uint64_t)gx * ((batch + 31u) / 32u) > 0x7fffffffull) return OXS_ERR_INVALID_ARGUMENT;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(64u * waves), 0, (hipStream_t)stream, y,
                        (const uint8_t*)w_packed, (const uint8_t*)x_q8_1, m, nb, batch, (batch + cols - 1u) / cols,

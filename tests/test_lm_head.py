@@ -196,6 +196,17 @@ def _to_dev(torch, arr):
     return torch.from_numpy(np.ascontiguousarray(arr)).cuda()
 
 
+def test_mmvq_refuses_more_workgroups_than_a_launch_holds():
+    # 128 tokens x 32 columns per workgroup: 2^24 x 2^7 of them are refused before anything is launched,
+    # however few workgroups the matrix kernel's larger forms would need
+    import ctypes
+    from oxide_sampler import _abi, load_library
+    lib = load_library()
+    p = ctypes.c_void_p(1 << 20)  # aligned, never read
+    assert lib.oxs_mmvq_q8_0(p, p, p, 1 << 31, 128, 128 * 32, None) == _abi.OXS_ERR_INVALID_ARGUMENT
+    assert lib.oxs_mmvq_q8_0(p, p, p, 1 << 31, 128, 128 * 32 * 4, None) == _abi.OXS_ERR_INVALID_ARGUMENT
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,k", [(1, 128), (3, 4096), (77, 896)])
 def test_gpu_quantize_matches_oracle(torch_gpu, batch, k):
