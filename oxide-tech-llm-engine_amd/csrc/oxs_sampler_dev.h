@@ -1156,7 +1156,7 @@ __device__ __forceinline__ uint32_t exact_select_row(const Params& p, const RowX
 // Bound: latency of one block's reads (16 per lane in flight) and the sort. The
 // radix select below reads the whole row five times or more and rebuilds its
 // penalty table per chunk and pass: 16 rows x 128256, top_k 1000, 512-id
-// windows took 787 to 835 us a call with it and take 192 with this.
+// windows took 803 us a call with it and take 184 with this.
 //
 // Returns M, with the keys sorted in area[kRecHash ...], or 0 where this does
 // not apply and nothing was written: DRY rows (their candidates predate DRY),

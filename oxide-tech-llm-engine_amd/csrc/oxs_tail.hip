@@ -1,11 +1,53 @@
 // oxs_tail.hip — the tail kernel (one block per row: top-M selection and the
 // chain) and the wide kernel (rows whose pool exceeds 1024), the second of
 // the sampler's launches.
+#include <stddef.h>
+
 #include <type_traits>
 
 #include "oxs_sampler_dev.h"
 
 namespace oxs {
+
+// The tail kernel's arguments, as they lie in memory.
+struct TailArgs {  // (tail_kernel's parameters in order)
+  const uint64_t *wave_theta, *lists;
+  const uint32_t* wave_count;
+  const uint64_t* libm;
+  uint32_t S, cap_w, cap_shift, rpx, B;
+  Params p;
+};
+
+template <typename T>
+__device__ __forceinline__ T* as_global(T* ptr) {
+  // (through an integer: a cast there and back alone is dropped, and the loads become flat ones)
+  return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)ptr;
+}
+
+// A copy of the launch parameters for a path that few rows take. The compiler loads the
+// arguments that any path uses at the kernel's entry and keeps them, spilled to
+// vector registers for want of scalar ones, through all of it; these come from
+// memory where they are used, so that they cost the other rows nothing.
+__device__ __forceinline__ Params late_params() {
+  typedef const __attribute__((address_space(4))) char* args_ptr;
+  args_ptr args = (args_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  Params q = *(const Params*)(const char*)(args + offsetof(TailArgs, p));
+  q.logits = as_global((const char*)q.logits);
+  q.configs = as_global(q.configs);
+  q.bias_ids = as_global(q.bias_ids);
+  q.bias_values = as_global(q.bias_values);
+  q.ban_ids = as_global(q.ban_ids);
+  q.mask = as_global(q.mask);
+  q.history = as_global(q.history);
+  q.logits_out = as_global(q.logits_out);
+  q.lists = as_global(q.lists);
+  q.wave_theta = as_global(q.wave_theta);
+  q.wave_count = as_global(q.wave_count);
+  q.dry_list = as_global(q.dry_list);
+  q.dry_count = as_global(q.dry_count);
+  return q;
+}
 
 // REC: rows whose candidates do not prove their top M try the wavefront
 // records before the radix select.
@@ -314,21 +356,23 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
     }
   }
   if (path == 2) {
-    const uint64_t* top = s_keys + kRecHash;
-    meff = 0;
+    const uint64_t* top = s_top;
     if constexpr (REC) {
-      meff = record_select_row<DT>(p, r, row, M, s_keys, &s_bstart_all[0][0], ts);
+      const Params q = late_params();
+      const RowIn in2 = load_row_in(q, row);
+      const RowXf r2 = make_row_xf_h(q, in2.cfg, in2.history_len);
+      meff = record_select_row<DT>(q, r2, row, M, s_keys, &s_bstart_all[0][0], ts);
       __syncthreads();  // (every wavefront has read what the attempt left in LDS)
+      if (meff) top = s_keys + kRecHash;
+      else meff = exact_select_row<DT>(q, r2, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
+    } else {
+      meff = exact_select_row<DT>(p, r, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
     }
     if (meff == 0) {
-      meff = exact_select_row<DT>(p, r, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
-      if (meff == 0) {
-        write_row_result<DT>(p, row, 0u, OXS_ROW_EMPTY, rs);
-        return;
-      }
-      bitonic_sort<false>(s_top, meff);
-      top = s_top;
+      write_row_result<DT>(p, row, 0u, OXS_ROW_EMPTY, rs);
+      return;
     }
+    if (top == s_top) bitonic_sort<false>(s_top, meff);
     keys_to_chain(top, meff, s_ids, s_pr, s_tab);
   }
 
@@ -433,9 +477,11 @@ static void launch_tail_rec(const Params& p, uint32_t grid_b, hipStream_t st) {
 
 // The record selection is compiled into the tail only where the sampler was
 // created for pools above 256 (max_top_k > 256): those rows need it on nearly
-// every call, while its mere presence costs every row 0.4 us (one row x 32000:
-// 12.9 -> 13.3, 24 x 50257: 17.0 -> 17.4), and rows of 256 keys rarely leave the
-// candidate path. Softcap and decode-step kinds keep the radix select alone.
+// every call, and rows of 256 keys rarely leave the candidate path. Softcap and
+// decode-step kinds keep the radix select alone. A row that does not need it pays
+// nothing for its presence: top_k 40, us without / with it and its arguments
+// kept from the kernel's entry / with late_params: 1 x 32000 12.67 / 12.84 / 12.78, 64 x
+// 128256 16.35 / 16.67 / 16.43, 256 x 128256 32.74 / 33.17 / 32.72.
 template <int KIND>
 static hipError_t launch_tail_k(const Params& p, uint32_t grid_b, hipStream_t st) {
   if constexpr (!kind_softcap(KIND) && !kind_decode(KIND)) {
