@@ -221,13 +221,17 @@ size_t oxs_sampler_workspace_bytes(const oxs_sampler* sampler);
  * row's top M = max(top_k, 256) candidates were found, for tests and tuning.
  * counts[OXS_PATH_BUCKETS]: a bucketed counting sort of the stream phase's
  * candidate keys (the fast path); [OXS_PATH_SORT]: a bitonic sort of those
- * keys (a bucket held too many); [OXS_PATH_EXACT]: a radix select over the
- * whole row (the candidates could not be proven to hold the top M, or the
- * row uses DRY); [OXS_PATH_NONE]: the row ended before the selection
- * (OXS_ROW_UNSUPPORTED, OXS_ROW_MISSING_STATE).
+ * keys (a bucket held too many); [OXS_PATH_EXACT]: the candidates could not
+ * be proven to hold the top M (or DRY may raise a value of the row): a radix
+ * select over the whole row, or, where the sampler's max_top_k is above 256, one more
+ * read of the part of the row that the stream phase's records leave open
+ * (oxs_sampler_record_rows: how many of the OXS_PATH_EXACT rows that settled);
+ * [OXS_PATH_NONE]: the row ended before the selection (OXS_ROW_UNSUPPORTED,
+ * OXS_ROW_MISSING_STATE).
  * oxs_sampler_count_paths turns the counting on (enable != 0) or off for later
- * calls and zeroes the counts; oxs_sampler_path_counts copies them out. Both
- * synchronise the device: not for the decode loop.
+ * calls and zeroes the counts; oxs_sampler_path_counts and
+ * oxs_sampler_record_rows copy them out. They synchronise the device: not for
+ * the decode loop.
  */
 #define OXS_PATH_BUCKETS 0
 #define OXS_PATH_SORT 1
@@ -235,6 +239,7 @@ size_t oxs_sampler_workspace_bytes(const oxs_sampler* sampler);
 #define OXS_PATH_NONE 3
 int oxs_sampler_count_paths(oxs_sampler* sampler, int enable);
 int oxs_sampler_path_counts(const oxs_sampler* sampler, uint32_t counts[4]);
+int oxs_sampler_record_rows(const oxs_sampler* sampler, uint32_t* rows);
 
 /*
  * Diagnostics: the read floor of the sampler's stream phase. Reads `batch`

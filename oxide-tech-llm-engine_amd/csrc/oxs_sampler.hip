@@ -332,7 +332,7 @@ struct oxs_sampler {
   uint32_t* dry_ghash;  // [max_batch][3][2 * dry_cap]
   uint32_t dry_cap;     // a row's DRY list entries: max_dry_ids kept to max_vocab, a power of two
   uint32_t* row_steps;  // [max_batch] decode steps each row has handed to the host
-  uint32_t* path_counts;  // [kPathKinds] rows per top-M selection path
+  uint32_t* path_counts;  // [kPathCounters] rows per top-M selection path
   uint64_t* wide_keys;    // rows with top_k > 1024 (max_top_k > 1024 only), else NULL
   uint32_t* wide_arr;
   uint32_t wide_n2, wide_ld;
@@ -356,7 +356,7 @@ struct Workspace {
   uint32_t* dry_ghash;    // [max_batch][3][2 * dry_cap], or null: DRY slices past kDryMax use the LDS hash
   uint32_t dry_cap;
   uint32_t* row_steps;    // [max_batch] (decode steps only; may be null otherwise)
-  uint32_t* path_counts;  // [kPathKinds] or null (counting off)
+  uint32_t* path_counts;  // [kPathCounters] or null (counting off)
   uint64_t* wide_keys;    // [max_batch][wide_n2] or null: rows with max(top_k, 256) > kMaxM are then unsupported
   uint32_t* wide_arr;     // [max_batch][7 * wide_ld]
   uint32_t wide_cap, wide_n2, wide_ld;
@@ -539,8 +539,8 @@ int oxs_sampler_create(oxs_sampler** out, const oxs_limits* limits, int device) 
                   hipMalloc((void**)&s->dry_count, B * sizeof(uint32_t)) == hipSuccess &&
                   hipMalloc((void**)&s->row_steps, B * sizeof(uint32_t)) == hipSuccess &&
                   hipMemset(s->row_steps, 0, B * sizeof(uint32_t)) == hipSuccess &&
-                  hipMalloc((void**)&s->path_counts, oxs::kPathKinds * sizeof(uint32_t)) == hipSuccess &&
-                  hipMemset(s->path_counts, 0, oxs::kPathKinds * sizeof(uint32_t)) == hipSuccess;
+                  hipMalloc((void**)&s->path_counts, oxs::kPathCounters * sizeof(uint32_t)) == hipSuccess &&
+                  hipMemset(s->path_counts, 0, oxs::kPathCounters * sizeof(uint32_t)) == hipSuccess;
   size_t b_wide = 0;
   if (ok && mtk > (uint32_t)oxs::kMaxM) {  // rows with top_k > 1024: the wide kernel's workspace
     uint32_t n2 = 1;
@@ -553,7 +553,7 @@ int oxs_sampler_create(oxs_sampler** out, const oxs_limits* limits, int device) 
   }
   s->bytes = b_lists + b_theta + b_count + oxs::kLibmWords * sizeof(uint64_t) +
              B * (dcap * (sizeof(uint64_t) + 6 * sizeof(uint32_t)) + 2 * sizeof(uint32_t)) +
-             oxs::kPathKinds * sizeof(uint32_t) +
+             oxs::kPathCounters * sizeof(uint32_t) +
              b_wide;
   if (ok) {  // the libm tables, as bit patterns, in the workspace
     uint64_t host[oxs::kLibmWords];
@@ -594,7 +594,7 @@ int oxs_sampler_count_paths(oxs_sampler* s, int enable) {
   if (!s) return OXS_ERR_INVALID_ARGUMENT;
   if (hipSetDevice(s->device) != hipSuccess) return OXS_ERR_HIP;
   if (hipDeviceSynchronize() != hipSuccess ||
-      hipMemset(s->path_counts, 0, oxs::kPathKinds * sizeof(uint32_t)) != hipSuccess ||
+      hipMemset(s->path_counts, 0, oxs::kPathCounters * sizeof(uint32_t)) != hipSuccess ||
       hipDeviceSynchronize() != hipSuccess)
     return OXS_ERR_HIP;
   s->count_paths = enable != 0;
@@ -606,6 +606,15 @@ int oxs_sampler_path_counts(const oxs_sampler* s, uint32_t* counts) {
   if (hipSetDevice(s->device) != hipSuccess) return OXS_ERR_HIP;
   if (hipDeviceSynchronize() != hipSuccess ||
       hipMemcpy(counts, s->path_counts, oxs::kPathKinds * sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
+    return OXS_ERR_HIP;
+  return OXS_OK;
+}
+
+int oxs_sampler_record_rows(const oxs_sampler* s, uint32_t* rows) {
+  if (!s || !rows) return OXS_ERR_INVALID_ARGUMENT;
+  if (hipSetDevice(s->device) != hipSuccess) return OXS_ERR_HIP;
+  if (hipDeviceSynchronize() != hipSuccess ||
+      hipMemcpy(rows, s->path_counts + oxs::kPathRecords, sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
     return OXS_ERR_HIP;
   return OXS_OK;
 }

@@ -95,7 +95,7 @@ struct Params {
   uint32_t* dec_count;    // [B] generated count
   uint64_t* host_tokens;  // [B] host memory: (row's step count << 32) | token
   uint32_t* row_steps;    // [B] workspace: decode steps each row has handed to the host
-  uint32_t* path_counts;  // [kPathKinds] workspace, or NULL: rows per top-M selection path
+  uint32_t* path_counts;  // [kPathCounters] workspace, or NULL: rows per top-M selection path
   // rows whose M = max(top_k, 256) exceeds kMaxM (the wide kernel), or NULL
   uint64_t* wide_keys;  // [B][wide_n2] a row's top-M keys, then sorted
   uint32_t* wide_arr;   // [B][7 * wide_ld] the chain's arrays of such a row
@@ -1507,9 +1507,11 @@ __device__ __forceinline__ void write_row_result(const Params& p, uint32_t row, 
 // counters are on (oxs_sampler_count_paths).
 constexpr int kPathBuckets = 0;  // bucketed counting sort of the candidate keys
 constexpr int kPathSort = 1;     // bitonic sort of the candidate keys
-constexpr int kPathExact = 2;    // radix select over the whole row
+constexpr int kPathExact = 2;    // the candidates do not prove the row's top M
 constexpr int kPathNone = 3;     // the row ended before the selection (unsupported, missing state)
-constexpr int kPathKinds = 4;
+constexpr int kPathKinds = 4;    // (oxs_sampler_path_counts)
+constexpr int kPathRecords = 4;  // of the exact ones, rows that the wavefront records settled
+constexpr int kPathCounters = 5;
 __device__ __forceinline__ void count_path(const Params& p, int path) {
   if (p.path_counts && threadIdx.x == 0) atomicAdd(&p.path_counts[path], 1u);
 }

@@ -363,8 +363,12 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
       const RowXf r2 = make_row_xf_h(q, in2.cfg, in2.history_len);
       meff = record_select_row<DT>(q, r2, row, M, s_keys, &s_bstart_all[0][0], ts);
       __syncthreads();  // (every wavefront has read what the attempt left in LDS)
-      if (meff) top = s_keys + kRecHash;
-      else meff = exact_select_row<DT>(q, r2, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
+      if (meff) {
+        count_path(q, kPathRecords);
+        top = s_keys + kRecHash;
+      } else {
+        meff = exact_select_row<DT>(q, r2, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
+      }
     } else {
       meff = exact_select_row<DT>(p, r, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
     }

@@ -203,6 +203,12 @@ class BatchSampler:
         check(self.lib.oxs_sampler_path_counts(self.handle, c), "oxs_sampler_path_counts")
         return {"buckets": int(c[0]), "sort": int(c[1]), "exact": int(c[2]), "none": int(c[3])}
 
+    def record_rows(self) -> int:
+        """How many of the `exact` rows the stream phase's records settled without a radix select."""
+        c = ctypes.c_uint32()
+        check(self.lib.oxs_sampler_record_rows(self.handle, ctypes.byref(c)), "oxs_sampler_record_rows")
+        return int(c.value)
+
     def launch(self, batch: OxsBatch, stream=None, decode: Optional[OxsDecodeIo] = None,
                no_alloc: bool = False) -> None:
         """Raw launch of a prepared descriptor on `stream` (torch stream or None);

@@ -296,6 +296,48 @@ def test_top_m_from_the_wavefront_records(torch_gpu, batch, vocab, dtype, kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("case", ["records", "wide rows beside it", "ids", "write-back", "dry", "few wavefronts",
+                                  "candidates"])
+def test_which_rows_the_records_settle(torch_gpu, case):
+    # pools of 1000 keys over 64 wavefronts of 128256 logits are settled by the wavefront records; a row
+    # falls through to the radix select with more than 1536 penalised ids, a write-back, DRY that can raise
+    # a value, wavefronts too few to bound 1000 keys (12 of 32 keys), or more than 2048 keys above the bound
+    # (every wavefront holds a run of equal values, larger than its list)
+    rng = np.random.default_rng(31)
+    B, V = 4, 3000 if case == "few wavefronts" else 128256
+    x = (rng.standard_normal((B, V)) * 3.0).astype(np.float32)
+    if case == "candidates":
+        x = np.minimum(x, 5.0)
+        x.reshape(B, -1, 16)[:, :, 0] = 5.0  # 8016 equal largest values
+    n = 1600 if case == "ids" else 500
+    hist = (rng.random((B, n)) * V).astype(np.uint32)
+    c = dict(repeat_penalty=1.2, repeat_last_n=0, temperature=1.0, top_k=1000, top_p=0.99)
+    if case == "dry":
+        hist[:, -8:-4] = hist[:, -4:]
+        c.update(dry_multiplier=0.8, dry_base=-1.2, dry_allowed_length=2)
+    configs = [wl.disabled_config(**c) for _ in range(B)]
+    if case == "wide rows beside it":
+        configs[1] = wl.disabled_config(**dict(c, top_k=1500))
+    w = wl.Workload(name=f"records: {case}", logits=x, dtype="f32", configs=configs, history=hist,
+                    history_len=np.full(B, n, np.uint32), uniforms=wl.xorshift_uniforms(B, 31))
+    banner(w.name)
+    from harness import gpu_sampler
+    most = 1500 if case == "wide rows beside it" else 1000
+    s = gpu_sampler(B, V, most, exact_limits=True)
+    s.count_paths(True)
+    try:
+        out = case == "write-back"
+        g = run_gpu(w, torch_gpu, kept_ld=most, record=False, max_top_k=most, exact_limits=True, logits_out=out)
+        counts, settled = s.path_counts(), s.record_rows()
+    finally:
+        s.count_paths(False)
+    print(counts, settled, flush=True)
+    compare(g, run_oracle(w, kept_ld=most, record=False, logits_out=out, n_threads=4), RTOL_F32, w.name)
+    assert counts["exact"] == B, counts
+    assert settled == {"records": B, "wide rows beside it": B - 1}.get(case, 0), settled
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("seed", range(5000, 5008))
 def test_random_decode_steps(torch_gpu, seed):
     # oxs_decode_step over three steps with random configs (raw-argmax rows included) and
