@@ -400,7 +400,8 @@ extern "C" int oxs_dfa_mask(const oxs_dfa* dfa, const oxs_token_bytes* tokens, c
   if ((dfa->num_states && !dfa->transitions) || !tokens->offsets || !tokens->bytes || !states || !mask)
     return OXS_ERR_INVALID_ARGUMENT;
   if (mask_ld < (int64_t)((tokens->vocab + 31u) / 32u)) return OXS_ERR_INVALID_ARGUMENT;
-  // token indices stay below 2^31; the batch within 65535 groups of 16 rows
+  // token indices stay below 2^31; at most 65535 x 16 rows, within the grid's y extent
+  // (a block covers 64 or 128)
   if (tokens->vocab > (1u << 31) || batch > 65535u * 16u) return OXS_ERR_INVALID_ARGUMENT;
   Params p;
   p.trans = dfa->transitions;

@@ -165,10 +165,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mmvq_q8_0_kernel(float* __restr
   constexpr int XR = (XW + kMmThreads - 1) / kMmThreads;
   // per group: quants as [k block][half g][column][16 bytes], then the scales
   // as [k block][column] pairs {half scale, 0}, as the matrix instruction
-  // takes them; after the two buffers, a third of zeros for lanes 32..63's scales
+  // takes them; after the two buffers, zeros for lanes 32..63's scales
   constexpr int XD = kGroupBlocks * 2 * PLANE * 4;
   constexpr int XG = XD + kGroupBlocks * COLS * 2;
-  __shared__ __align__(16) uint32_t s_x[2 * XG + XG];
+  __shared__ __align__(16) uint32_t s_x[2 * XG + (XG - XD)];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   // token block tb and column block cb: in each run of 8 * ncb workgroups,
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mmvq_q8_0_kernel(float* __restr
   const uint32_t c0 = cb * COLS;
   const uint32_t ngroups = nb / kGroupBlocks;
 
-  // staging: dword i of a group's COLS x 36 dwords, for i = tid, tid + 512, ...:
+  // staging: dword i of a group's COLS x 36 dwords, for i = tid, tid + kMmThreads, ...:
   // consecutive lanes read consecutive dwords of a column's 144 bytes
   // (offsets from the column block; 32 bits for 64 columns, which the host
   // takes only where they suffice)
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mmvq_q8_0_kernel(float* __restr
   // zeros: the scales' second words, which staging never writes, and lanes 32..63's scales
   for (uint32_t i = tid; i < 2u * kGroupBlocks * COLS; i += kMmThreads)
     s_x[(i / (kGroupBlocks * COLS)) * XG + XD + (i % (kGroupBlocks * COLS)) * 2u + 1u] = 0u;
-  for (uint32_t i = tid; i < (uint32_t)XG; i += kMmThreads) s_x[2 * XG + i] = 0u;
+  for (uint32_t i = tid; i < (uint32_t)(XG - XD); i += kMmThreads) s_x[2 * XG + i] = 0u;
   stage_store(0);
   __syncthreads();
   uint32_t buf = 0;
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mmvq_q8_0_kernel(float* __restr
     const uint8_t* next = group_at(grp + PF);
     const uint32_t* xg = s_x + buf * XG;
     const uint32_t* xq = xg + (g * PLANE + j) * 4u;
-    const uint32_t* xd = (g ? s_x + 2 * XG : xg) + XD + 2u * j;
+    const uint32_t* xd = (g ? s_x + 2 * XG : xg + XD) + 2u * j;
     // a tile's columns are read from LDS one tile ahead
     uint4 bq;
     uint64_t dx;
