@@ -601,22 +601,30 @@ int oxs_sampler_count_paths(oxs_sampler* s, int enable) {
   return OXS_OK;
 }
 
-int oxs_sampler_path_counts(const oxs_sampler* s, uint32_t* counts) {
-  if (!s || !counts) return OXS_ERR_INVALID_ARGUMENT;
+static int read_path_counters(const oxs_sampler* s, uint32_t (&c)[oxs::kPathCounters]) {
   if (hipSetDevice(s->device) != hipSuccess) return OXS_ERR_HIP;
   if (hipDeviceSynchronize() != hipSuccess ||
-      hipMemcpy(counts, s->path_counts, oxs::kPathKinds * sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
+      hipMemcpy(c, s->path_counts, sizeof(c), hipMemcpyDeviceToHost) != hipSuccess)
     return OXS_ERR_HIP;
+  return OXS_OK;
+}
+
+int oxs_sampler_path_counts(const oxs_sampler* s, uint32_t* counts) {
+  if (!s || !counts) return OXS_ERR_INVALID_ARGUMENT;
+  uint32_t c[oxs::kPathCounters];
+  const int rc = read_path_counters(s, c);
+  if (rc != OXS_OK) return rc;
+  for (int i = 0; i < oxs::kPathKinds; ++i) counts[i] = c[i];
+  counts[oxs::kPathExact] += c[oxs::kPathNoRecords];
   return OXS_OK;
 }
 
 int oxs_sampler_record_rows(const oxs_sampler* s, uint32_t* rows) {
   if (!s || !rows) return OXS_ERR_INVALID_ARGUMENT;
-  if (hipSetDevice(s->device) != hipSuccess) return OXS_ERR_HIP;
-  if (hipDeviceSynchronize() != hipSuccess ||
-      hipMemcpy(rows, s->path_counts + oxs::kPathRecords, sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
-    return OXS_ERR_HIP;
-  return OXS_OK;
+  uint32_t c[oxs::kPathCounters];
+  const int rc = read_path_counters(s, c);
+  if (rc == OXS_OK) *rows = c[oxs::kPathExact] - c[oxs::kPathFellThrough];
+  return rc;
 }
 
 }  // extern "C"

@@ -1141,6 +1141,24 @@ __device__ __forceinline__ uint32_t exact_select_row(const Params& p, const RowX
   return meff;
 }
 
+// Which way a row's top M was found, counted per row when the sampler's path
+// counters are on (oxs_sampler_count_paths).
+constexpr int kPathBuckets = 0;  // bucketed counting sort of the candidate keys
+constexpr int kPathSort = 1;     // bitonic sort of the candidate keys
+constexpr int kPathExact = 2;    // the candidates do not prove the row's top M
+constexpr int kPathNone = 3;     // the row ended before the selection (unsupported, missing state)
+constexpr int kPathKinds = 4;    // (oxs_sampler_path_counts)
+// Exact rows are counted apart where no record selection is compiled in (and in the
+// wide kernel), and where one fell through, so that the rows it settled follow
+// without a counter on their way: one there cost 4.5 us of 191, by the code
+// it made of the loops around it.
+constexpr int kPathNoRecords = 4;
+constexpr int kPathFellThrough = 5;
+constexpr int kPathCounters = 6;
+__device__ __forceinline__ void count_path(const Params& p, int path) {
+  if (p.path_counts && threadIdx.x == 0) atomicAdd(&p.path_counts[path], 1u);
+}
+
 // The row's top M where the candidate keys alone do not prove it: a pool of
 // more than 256 keys (top_k > 256), or a wavefront whose list or whose chunk's
 // hash overflowed. The stream kernel's records still bound the M-th key from
@@ -1501,19 +1519,6 @@ __device__ __forceinline__ void write_row_result(const Params& p, uint32_t row, 
     if (p.out_kept_count && !rs.raw) p.out_kept_count[row] = 0;
     decode_advance<DT>(p, row, token, rs);
   }
-}
-
-// Which way a row's top M was found, counted per row when the sampler's path
-// counters are on (oxs_sampler_count_paths).
-constexpr int kPathBuckets = 0;  // bucketed counting sort of the candidate keys
-constexpr int kPathSort = 1;     // bitonic sort of the candidate keys
-constexpr int kPathExact = 2;    // the candidates do not prove the row's top M
-constexpr int kPathNone = 3;     // the row ended before the selection (unsupported, missing state)
-constexpr int kPathKinds = 4;    // (oxs_sampler_path_counts)
-constexpr int kPathRecords = 4;  // of the exact ones, rows that the wavefront records settled
-constexpr int kPathCounters = 5;
-__device__ __forceinline__ void count_path(const Params& p, int path) {
-  if (p.path_counts && threadIdx.x == 0) atomicAdd(&p.path_counts[path], 1u);
 }
 
 // LDS arrays of the chain; each is readable 16 entries past kMaxM.

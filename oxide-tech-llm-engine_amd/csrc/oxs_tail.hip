@@ -46,6 +46,7 @@ __device__ __forceinline__ Params late_params() {
   q.wave_count = as_global(q.wave_count);
   q.dry_list = as_global(q.dry_list);
   q.dry_count = as_global(q.dry_count);
+  q.path_counts = as_global(q.path_counts);
   return q;
 }
 
@@ -269,7 +270,8 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
   const bool linear = !exact && kmax >= theta_max && range > 0.0f && range <= __FLT_MAX__ &&
                       scale <= __FLT_MAX__ && vmax <= __FLT_MAX__ && vmin >= -__FLT_MAX__;
   uint32_t meff = 0;
-  int path = exact ? 2 : 1;  // 0 buckets, 1 sort, 2 exact re-scan
+  constexpr int kExact = REC ? kPathExact : kPathNoRecords;
+  int path = exact ? kExact : 1;  // 0 buckets, 1 sort, kExact exact re-scan
   uint32_t bs[PER];
   uint32_t* s_bstart = s_bstart_all[wave];
   uint32_t last = 0;
@@ -300,7 +302,7 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
     if (st2 < meff && st2 + c4.z >= meff) mine = lane * 4 + 2;
     if (st3 < meff && st3 + c4.w >= meff) mine = lane * 4 + 3;
     last = wave_reduce32(mine, MinOp{});  // the bucket of the meff-th key
-    if (N < M && !all_kept) path = 2;
+    if (N < M && !all_kept) path = kExact;
     else if (big > kBigBucket) path = 1;
     else path = 0;
     wave_sync();
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
     __syncthreads();
   } else if (path == 1) {
     const uint32_t N = sort_select(yk, vm, M, s_keys, s_top, ts);
-    if (N < M && !all_kept) path = 2;
+    if (N < M && !all_kept) path = kExact;
     count_path(p, path);
     if (path == 1) {
       meff = min(M, N);
@@ -355,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
       keys_to_chain(s_top, meff, s_ids, s_pr, s_tab);
     }
   }
-  if (path == 2) {
+  if (path == kExact) {
     const uint64_t* top = s_top;
     if constexpr (REC) {
       const Params q = late_params();
@@ -364,9 +366,9 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(const uint64_t* __restri
       meff = record_select_row<DT>(q, r2, row, M, s_keys, &s_bstart_all[0][0], ts);
       __syncthreads();  // (every wavefront has read what the attempt left in LDS)
       if (meff) {
-        count_path(q, kPathRecords);
         top = s_keys + kRecHash;
       } else {
+        count_path(q, kPathFellThrough);
         meff = exact_select_row<DT>(q, r2, row, M, (uint32_t*)s_keys, s_bcount, s_top, ts);
       }
     } else {
@@ -443,7 +445,7 @@ __global__ __launch_bounds__(kThreads) void wide_kernel(const Params p) {
     write_row_result<DT>(p, row, 0u, OXS_ROW_UNSUPPORTED, rs);
     return;
   }
-  count_path(p, kPathExact);
+  count_path(p, kPathNoRecords);
   uint64_t* keys = p.wide_keys + (size_t)row * p.wide_n2;
   const uint32_t meff = exact_select_row<DT>(p, r, row, M, (uint32_t*)s_area, s_hist, keys, ts, p.wide_cap);
   if (meff == 0) {
