@@ -463,9 +463,9 @@ __device__ uint32_t block_excl_scan(uint32_t v, uint32_t* total, uint32_t* scrat
 // constant, that falls through: with many blocks this kernel is bound by instruction
 // issue, and about 20 instructions per wavefront are 2% of it.
 // Measured, us, one table of 256 / 256 to 960 slots by the row's ids, scaled / this:
-// 256 rows x 151936 bf16, 256 ids 36.1 / 37.0 / 36.3, 513 ids 39.3 / 39.1 / 38.8;
-// 512 x 262144, 300 ids 92.8 / 94.7 / 93.3; 64 x 128256, 512 ids 20.4 / 17.2 / 17.3;
-// 64 x 128256, 900 distinct ids in one chunk 780 / 38 / 23.
+// 256 rows x 151936 bf16, 256 ids 36.1 / 37.0 / 36.5, 513 ids 39.3 / 39.3 / 39.0;
+// 512 x 262144, 300 ids 92.4 / 94.3 / 92.9; 64 x 128256, 512 ids over the vocabulary
+// 16.4 / 16.6 / 16.7, skewed 20.5 / 17.3 / 17.4; 900 distinct ids in one chunk 780 / 38 / 23.
 // 1024 slots beside the 32 KB of staged values are a quarter of the CU's 160 KB of
 // LDS, so four blocks stay resident; the overflow mark is the last slot's value.
 constexpr uint32_t kHashBits = 10;
@@ -493,9 +493,13 @@ __device__ __forceinline__ uint32_t hash_slot(uint32_t key, uint32_t bits) {
 }
 
 // Continues an insertion whose home slot held another key; false when `probes` slots held others.
+// (A launch of few rounds of blocks pays for its code's length: unrolled 8 times at each of its
+// eight uses, the larger table's probes cost 64 x 128256 rows of 512 ids 0.2 us.)
+template <int UNROLL>
 __device__ __forceinline__ bool hash_insert_from(uint32_t* hkeys, uint32_t* hvals, uint32_t bits, uint32_t probes,
                                                  uint32_t key, uint32_t add, uint32_t orv) {
   uint32_t h = hash_slot(key, bits);
+#pragma unroll UNROLL
   for (uint32_t probe = 0; probe < probes; ++probe) {
     const uint32_t prev = atomicCAS(&hkeys[h], kEmptySlot, key);
     if (prev == kEmptySlot || prev == key) {
@@ -529,7 +533,7 @@ __device__ __forceinline__ void build_marks(const Params& p, const RowXf& r, uin
   const uint32_t probes = BITS || ids < 1u << bits ? 1u << bits : kHashProbes;
   bool ok = true;
   const auto insert = [&](uint32_t key, uint32_t add, uint32_t orv) {
-    ok &= hash_insert_from(s_hkeys, s_hvals, bits, probes, key, add, orv);
+    ok &= hash_insert_from<BITS ? 8 : 4>(s_hkeys, s_hvals, bits, probes, key, add, orv);
   };
   uint32_t prev[kHistUnroll];
 #pragma unroll
@@ -590,7 +594,7 @@ __device__ __forceinline__ void rebuild_marks(const Params& p, const RowXf& r, u
     if (j < wn) id = p.history[(size_t)row * p.history_ld + r.wstart + j], flag = 0u;
     else if (j < n1) id = p.ban_ids[r.ban_off + (j - wn)], flag = kBanFlag;
     else if (j < n2) id = p.bias_ids[r.bias_off + (j - n1)], flag = kBiasFlag;
-    if (id >= c0 && id < c1) hash_insert_from(s_hkeys, s_hvals, kHashBits, kHashSlots, id - c0, flag ? 0u : 1u, flag);
+    if (id >= c0 && id < c1) hash_insert_from<1>(s_hkeys, s_hvals, kHashBits, kHashSlots, id - c0, flag ? 0u : 1u, flag);
   }
   __syncthreads();
 }
@@ -656,19 +660,25 @@ __device__ __forceinline__ void process_unit(const Params& p, uint32_t row, uint
     // the slots of a thread: one, or two or four in a row
     uint32_t h = tid, turns = 1;
     uint4 k;
-    if (__builtin_expect(ids > kHashSmall, 0)) {
-      uint32_t bits = hash_bits_of(ids);
-      if (ids <= kHashTryMid && *s_full != 0u) {
-        __syncthreads();  // (every wavefront has read the mark)
-        rebuild_marks(p, r, row, c0, c1, s_hkeys, s_hvals);
-        bits = kHashBits;
-      }
-      turns = 1u << (bits - 8u);
+    if (__builtin_expect(ids > kHashTry, 0)) {
+      const bool mid = ids <= kHashTryMid;
+      k = *(const uint4*)&s_hkeys[mid ? (2u * tid) & ~3u : 4u * tid];
+      const uint32_t full = *s_full;  // (one wait for both)
+      turns = mid ? 2u : 4u;
       h = tid * turns;
-      if (bits > 8u) k = *(const uint4*)&s_hkeys[bits == 9u ? h & ~3u : h];
-      if (bits == 9u && (tid & 1u)) k.x = k.z, k.y = k.w;
+      if (mid && (tid & 1u)) k.x = k.z, k.y = k.w;
+      if (mid && full != 0u) turns = 0u;
+    } else {
+      k.x = s_hkeys[tid];
+      if (__builtin_expect(ids > kHashSmall, 0) && *s_full != 0u) turns = 0u;
     }
-    if (turns == 1u) k.x = s_hkeys[tid];
+    if (__builtin_expect(turns == 0u, 0)) {
+      __syncthreads();  // (every wavefront has read the mark)
+      rebuild_marks(p, r, row, c0, c1, s_hkeys, s_hvals);
+      turns = 4u;
+      h = 4u * tid;
+      k = *(const uint4*)&s_hkeys[h];
+    }
 #pragma unroll 1
     do {  // (block-uniform turns)
       const uint32_t off = k.x;
@@ -1227,17 +1237,17 @@ __device__ __forceinline__ uint32_t record_select_row(const Params& p, const Row
   if (r.use_hist) {
     const uint32_t* win = p.history + (size_t)row * p.history_ld + r.wstart;
     for (uint32_t j = tid; j < r.wn; j += kThreads)
-      if (win[j] < p.V) hash_insert_from(hk, hv, kRecBits, kRecHash, win[j], 1u, 0u);
+      if (win[j] < p.V) hash_insert_from<2>(hk, hv, kRecBits, kRecHash, win[j], 1u, 0u);
   }
   for (uint32_t k = tid; k < r.ban_cnt; k += kThreads) {
     const uint32_t id = p.ban_ids[r.ban_off + k];
-    if (id < p.V) hash_insert_from(hk, hv, kRecBits, kRecHash, id, 0u, kBanFlag);
+    if (id < p.V) hash_insert_from<2>(hk, hv, kRecBits, kRecHash, id, 0u, kBanFlag);
   }
   for (uint32_t k = tid; k < r.bias_cnt; k += kThreads) {
     const uint32_t id = p.bias_ids[r.bias_off + k];
-    if (id < p.V) hash_insert_from(hk, hv, kRecBits, kRecHash, id, 0u, kBiasFlag);
+    if (id < p.V) hash_insert_from<2>(hk, hv, kRecBits, kRecHash, id, 0u, kBiasFlag);
   }
-  if (tid == 0 && r.nl_active) hash_insert_from(hk, hv, kRecBits, kRecHash, r.nl_id, 0u, kNlFlag);
+  if (tid == 0 && r.nl_active) hash_insert_from<2>(hk, hv, kRecBits, kRecHash, r.nl_id, 0u, kNlFlag);
   __syncthreads();
   const auto push = [&](uint64_t key) {
     const uint32_t q = atomicAdd(&ts.counter, 1u);
