@@ -139,20 +139,20 @@ def test_random_configs_large_vocab(torch_gpu, seed):
 
 @pytest.mark.gpu
 def test_logits_out_when_penalty_ids_overflow_the_chunk_hash(torch_gpu):
-    # V = 1000 is one stream chunk; a whole-history window of 900 distinct ids overflows its
-    # 256-slot LDS hash, so the row goes to the exact path, which must write every id of
-    # logits_out with its penalties (sampler.rs:207-245)
+    # V = 1024 is one stream chunk; a whole-history window of all of its ids overflows its hash (1023
+    # ids), so the row goes to the exact path, which must write every id of logits_out with its
+    # penalties (sampler.rs:207-245)
     rng = np.random.default_rng(77)
-    B, V = 4, 1000
+    B, V = 4, 1024
     logits = (rng.standard_normal((B, V)) * 2.0).astype(np.float32)
-    history = np.stack([rng.permutation(V)[:900].astype(np.uint32) for _ in range(B)])
+    history = np.stack([rng.permutation(V)[:1024].astype(np.uint32) for _ in range(B)])
     configs = [wl.disabled_config(frequency_penalty=0.6, presence_penalty=0.2, repeat_last_n=0),
                wl.disabled_config(repeat_penalty=1.3, repeat_last_n=0, temperature=0.7),
                wl.disabled_config(presence_penalty=-0.2, top_k=40, top_p=0.9),
-               wl.disabled_config(frequency_penalty=0.3, repeat_penalty=1.1, repeat_last_n=900, min_p=0.05)]
+               wl.disabled_config(frequency_penalty=0.3, repeat_penalty=1.1, repeat_last_n=1024, min_p=0.05)]
     w = wl.Workload(name="hash overflow", logits=logits, dtype="f32", configs=configs, history=history,
-                    history_len=np.full(B, 900, np.uint32), uniforms=wl.xorshift_uniforms(B, 77))
-    banner("logits_out with 900 distinct penalty ids in one chunk")
+                    history_len=np.full(B, 1024, np.uint32), uniforms=wl.xorshift_uniforms(B, 77))
+    banner("logits_out with 1024 distinct penalty ids in one chunk")
     g = run_gpu(w, torch_gpu, logits_out=True, record=False)
     r = run_oracle(w, logits_out=True, record=False)
     compare(g, r, RTOL_F32, w.name)
@@ -161,8 +161,8 @@ def test_logits_out_when_penalty_ids_overflow_the_chunk_hash(torch_gpu):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [255, 256, 257, 320, 321, 960, 961, 1024])
 def test_penalty_ids_at_the_sizes_of_the_chunk_hash(torch_gpu, n):
-    # n distinct window ids in one stream chunk: the hash takes 256 slots, then steps of 64 up to
-    # 960, exactly full at 256, 320 and 960; from 961 on it overflows and the row is re-scanned
+    # n distinct window ids in one stream chunk: its hash takes 256 slots (built again in 1024 where they
+    # do not suffice), 512 or 1024 by the row's ids, full at 256, 512 and 1023
     rng = np.random.default_rng(n)
     B, V = 3, 1024
     logits = (rng.standard_normal((B, V)) * 2.0).astype(np.float32)
